@@ -141,8 +141,8 @@ struct SolveTasks {
 struct StepPlan {
   int32_t k0;
   int64_t panel_off, panel_cnt;  // front ids
-  int64_t rows_off, rows_cnt;    // (front, row0): update rows s..f-1 of the panel, 64 per task
-  int64_t trsm_off, trsm_cnt;    // (front, col0)
+  int32_t rows;                  // most pivot candidates of a front in this step
+  int64_t apply_off, apply_cnt;  // (front, position, kind): 64 update rows (0) or columns outside the panel (1)
   int64_t gemm_off, gemm_cnt;    // (front, row0, col0)
 };
 struct LevelSched {

@@ -197,21 +197,17 @@ void devmesh_build(DevMesh &dm, hipStream_t s) {
       for (int32_t t : LP.fronts)
         if (sy.fronts[t].s > k0) tasks.push_back(t);
       st.panel_cnt = (int64_t)tasks.size() - st.panel_off;
-      st.rows_off = (int64_t)tasks.size();
+      st.rows = LP.max_s - k0;
+      st.apply_off = (int64_t)tasks.size();
       for (int32_t t : LP.fronts) {
         const FrontInfo &F = sy.fronts[t];
         if (F.s <= k0) continue;
-        for (int32_t r = F.s; r < F.f; r += 64) { tasks.push_back(t); tasks.push_back(r); }
+        const int32_t ke = k0 + std::min(NBP, F.s - k0);
+        for (int32_t r = F.s; r < F.f; r += 64) tasks.insert(tasks.end(), {t, r, 0});
+        for (int32_t c = ke; c < F.f; c += 64) tasks.insert(tasks.end(), {t, c, 1});
+        for (int32_t c = 0; c < k0; c += 64) tasks.insert(tasks.end(), {t, c, 1});
       }
-      st.rows_cnt = ((int64_t)tasks.size() - st.rows_off) / 2;
-      st.trsm_off = (int64_t)tasks.size();
-      for (int32_t t : LP.fronts) {
-        const FrontInfo &F = sy.fronts[t];
-        if (F.s <= k0) continue;
-        int32_t ke = k0 + std::min(NBP, F.s - k0);
-        for (int32_t c = ke; c < F.f; c += 64) { tasks.push_back(t); tasks.push_back(c); }
-      }
-      st.trsm_cnt = ((int64_t)tasks.size() - st.trsm_off) / 2;
+      st.apply_cnt = ((int64_t)tasks.size() - st.apply_off) / 3;
       st.gemm_off = (int64_t)tasks.size();
       for (int32_t t : LP.fronts) {
         const FrontInfo &F = sy.fronts[t];
