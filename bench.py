@@ -288,7 +288,7 @@ def trace_summary(trace_dir, top=30):
 def trace_levels(trace_dir, workdir):
     """Factorisation time and TFLOP/s by elimination-tree level from a
     rocprofv3 --kernel-trace CSV of the bench: each stream's kernels from
-    k_scatter_fronts to k_triinv are one factorisation, split into levels
+    k_scatter_fronts to k_tri_diag are one factorisation, split into levels
     (leaves first) after each level's k_extend_add launches; flops from the
     symbolic count of the bench meshes (averaged over the three)."""
     import csv
@@ -298,7 +298,7 @@ def trace_levels(trace_dir, workdir):
     files = glob.glob(os.path.join(trace_dir, '**', '*kernel_trace.csv'), recursive=True)
     if not files:
         raise SystemExit('no kernel_trace.csv under %s' % trace_dir)
-    lu = ('k_scatter_fronts', 'k_panel', 'k_trsm', 'k_panel_rows', 'k_gemm_update', 'k_extend_add')
+    lu = ('k_scatter_fronts', 'k_panel', 'k_gemm_update', 'k_extend_add')
     streams = collections.defaultdict(list)
     with open(files[0]) as f:
         for r in csv.DictReader(f):
@@ -312,7 +312,7 @@ def trace_levels(trace_dir, workdir):
             if n.startswith('k_scatter_fronts'):
                 cur = dict(nb=gy, levels=[[]])
                 facts.append(cur)
-            elif cur is not None and (n.startswith('k_triinv') or n.startswith('k_gather_index')):
+            elif cur is not None and (n.startswith('k_tri_diag') or n.startswith('k_gather_index')):
                 cur = None
             elif cur is not None and any(n.startswith(x) for x in lu):
                 lv = cur['levels']

@@ -439,7 +439,7 @@ void solve_dense(Ctx *c, int nb, int n, const zd *M, const zd *R, int r, zd *X) 
   int32_t *sig = c->buf<int32_t>("ds_sig", (size_t)nb * n);
   int32_t *gx = c->buf<int32_t>("ds_gx", (size_t)nb * n * 4);
   zd *inv = c->buf<zd>("ds_inv", (size_t)nb * dm.isz);
-  lu_factor(dm, nb, M, pool, piv, pfl, sig, gx, inv, s);
+  lu_factor(dm, nb, M, pool, piv, pfl, sig, gx, inv, c->buf<zd>("ds_inv_w", (size_t)nb * dm.wsz), s);
   const zd *rhs = R;
   if (!R) {
     zd *I = c->buf<zd>("ds_eye", (size_t)nb * n * n);

@@ -159,6 +159,19 @@ struct LevelSched {
   double fwd_mat = 0, fwd_vec = 0, bwd_mat = 0, bwd_vec = 0;
 };
 
+// One 64 x 64 tile of a product of the factor inversion, C = A B (-A B: neg;
+// added to C: acc): A is M x K (ld lda), B K x N, C M x N, at offsets into an instance's
+// front pool (base 0), inverted form (1) or intermediate products (2).  tri:
+// A holds another triangle beyond the diagonal k = m + doff; 1: unit lower, 2:
+// upper.
+struct InvTile {
+  int64_t aoff, boff, coff;
+  int32_t lda, ldb, ldc, M, N, K;
+  int16_t abase, bbase, cbase, neg, acc, tri;
+  int32_t doff;
+};
+static_assert(sizeof(InvTile) == 64, "InvTile is 16 words");
+
 struct DevMesh {
   Mesh host;
   int64_t ntyp = 0;
@@ -189,10 +202,12 @@ struct DevMesh {
   int64_t isz = 0;                   // inverted-form entries per instance
   int64_t part_rhs = 0;              // partial-sum entries per RHS (largest level)
   DBuf<int32_t> tasks;               // all task lists
-  int64_t tri_off = 0, tri_cnt = 0;  // triangular inversion tasks (front, J, kind)
-  int64_t wz_off = 0, wz_cnt = 0;    // off-diagonal inverted blocks (front, kind, row0, col0)
+  int64_t tri_off = 0, tri_cnt = 0;  // diagonal blocks of the triangular inversion (front, J, kind)
+  DBuf<InvTile> inv_tiles;           // its products, in dependent phases (first tile, count)
+  std::vector<std::pair<int64_t, int64_t>> inv_phases;
+  int64_t wsz = 0;                   // entries of their intermediate products per instance
   std::vector<LevelSched> sched;     // sched[0] = deepest level
-  int32_t max_f = 0;
+  int32_t max_f = 0, max_s = 0;
   // geometry for the plane-wave integrals
   // 1D gratings
   DBuf<double> h1d, xd1d, tab1d;     // element lengths, DOF coordinates (nel x 11), integral tables
@@ -260,11 +275,11 @@ void launch_permute_vals(DevMesh &dm, int nb, const zd *src, zd *dst, hipStream_
 // ---------------- LU kernels (kernels_lu.hip) ----------------
 // numeric factorisation into pool (piv: LAPACK-style row swaps, pflag: zero
 // pivots perturbed, sig: pivot-order gather), then the inverted-factor form
-// inv [nb][isz] and the forward gather records gx [nb][npiv][4] (per pivot:
+// inv [nb][isz] (wt [nb][wsz]: its intermediate products) and the forward gather records gx [nb][npiv][4] (per pivot:
 // right-hand-side index, the two child update entries) that the solves read
 void lu_factor(DevMesh &dm, int nb, const zd *mat1, zd *pool, int32_t *piv, int32_t *pflag, int32_t *sig,
-               int32_t *gx, zd *inv, hipStream_t s);
-void lu_invert(DevMesh &dm, int nb, const zd *pool, zd *inv, hipStream_t s);
+               int32_t *gx, zd *inv, zd *wt, hipStream_t s);
+void lu_invert(DevMesh &dm, int nb, const zd *pool, zd *inv, zd *wt, hipStream_t s);
 // x = A^{-1} b, both in the new (nested-dissection) numbering, [nb][nrhs][n];
 // y (same shape) and w ([nb][nrhs][solve_ws(dm)]) are work vectors.  sx:
 // instance stride of x (default nrhs n), so that x can be a column slot of a

@@ -165,6 +165,7 @@ void devmesh_build(DevMesh &dm, hipStream_t s) {
   dm.pmap.upload(sy.pmap, s);
   dm.nnz2front.upload(sy.nnz2front, s);
   dm.max_f = sy.max_f;
+  dm.max_s = nf ? *std::max_element(fs.begin(), fs.end()) : 0;
   // inverted-factor form: per front the offset of its forward / backward
   // blocks (2 f s entries) and of its rows in the child update-vector map
   std::vector<int64_t> io(nf), fv(nf);
@@ -323,22 +324,79 @@ void devmesh_build(DevMesh &dm, hipStream_t s) {
     dm.tri_off = (int64_t)tasks.size();
     for (int32_t i = 0; i < nf; ++i)
       for (int kind = 0; kind < 2; ++kind)
-        for (int32_t J = 0; J < (sy.fronts[i].s + 31) / 32; ++J) {
-          tasks.push_back(i); tasks.push_back(J); tasks.push_back(kind);
-        }
+        for (int32_t J = 0; J < (sy.fronts[i].s + TL - 1) / TL; ++J) tasks.insert(tasks.end(), {i, J, kind});
     dm.tri_cnt = ((int64_t)tasks.size() - dm.tri_off) / 3;
-    dm.wz_off = (int64_t)tasks.size();
+    // products of the inversion: for h = 64, 128, ... the off-diagonal block
+    // X of every pair of inverted diagonal blocks A = [i0, i0 + h) and C = the
+    // next min(h, s - i0 - h) rows: W = B A^-1, X = -C^-1 W, and the residual
+    // correction W += C X, X -= C^-1 W (lower; upper: W = B C^-1, X = -A^-1 W,
+    // W += A X, X -= A^-1 W); last the off-diagonal blocks of the inverted
+    // form.  Triangular operands are read only inside their triangle.
+    std::vector<InvTile> tiles;
+    auto tile = [&](int M, int N, int r, int c, int k0, int k1, int ab, int64_t ao, int la, int bb, int64_t bo,
+                    int lb, int cb, int64_t co, int lc, int neg, int acc = 0, int tri = 0) {
+      InvTile T{};
+      T.aoff = ao + r + (int64_t)k0 * la;
+      T.boff = bo + k0 + (int64_t)c * lb;
+      T.coff = co + r + (int64_t)c * lc;
+      T.lda = la; T.ldb = lb; T.ldc = lc;
+      T.M = std::min(TL, M - r); T.N = std::min(TL, N - c); T.K = k1 - k0;
+      T.abase = (int16_t)ab; T.bbase = (int16_t)bb; T.cbase = (int16_t)cb; T.neg = (int16_t)neg; T.acc = (int16_t)acc; T.tri = (int16_t)tri; T.doff = r - k0;
+      tiles.push_back(T);
+    };
+    for (int32_t h = TL; h < dm.max_s; h *= 2)
+      for (int ph = 0; ph < 4; ++ph) {
+        const int64_t first = (int64_t)tiles.size();
+        int64_t wo = 0;
+        for (int32_t i = 0; i < nf; ++i) {
+          const FrontInfo &F = sy.fronts[i];
+          for (int kind = 0; kind < 2; ++kind)
+            for (int32_t i0 = 0; i0 + h < F.s; i0 += 2 * h) {
+              const int32_t i1 = i0 + h, cn = std::min(h, F.s - i1), f = F.f, sn = F.s;
+              const int64_t O0 = io[i], O1 = io[i] + (int64_t)f * sn;
+              const int32_t M = kind ? h : cn, N = kind ? cn : h;
+              for (int32_t r = 0; r < M; r += TL)
+                for (int32_t c = 0; c < N; c += TL) {
+                  if (ph == 0 && kind == 0)
+                    tile(M, N, r, c, c, h, 0, F.off + i1 + (int64_t)i0 * f, f, 1, O0 + i0 + (int64_t)i0 * f, f, 2, wo,
+                         M, 0);
+                  else if (ph == 0)
+                    tile(M, N, r, c, 0, std::min(cn, c + TL), 0, F.off + i0 + (int64_t)i1 * f, f, 1,
+                         O1 + i1 + (int64_t)i1 * sn, sn, 2, wo, M, 0);
+                  else if (ph == 2 && kind == 0)
+                    tile(M, N, r, c, 0, std::min(cn, r + TL), 0, F.off + i1 + (int64_t)i1 * f, f, 1,
+                         O0 + i1 + (int64_t)i0 * f, f, 2, wo, M, 0, 1, 1);
+                  else if (ph == 2)
+                    tile(M, N, r, c, r, h, 0, F.off + i0 + (int64_t)i0 * f, f, 1, O1 + i0 + (int64_t)i1 * sn, sn, 2, wo,
+                         M, 0, 1, 2);
+                  else if (kind == 0)
+                    tile(M, N, r, c, 0, std::min(cn, r + TL), 1, O0 + i1 + (int64_t)i1 * f, f, 2, wo, M, 1,
+                         O0 + i1 + (int64_t)i0 * f, f, 1, ph == 3);
+                  else
+                    tile(M, N, r, c, r, h, 1, O1 + i0 + (int64_t)i0 * sn, sn, 2, wo, M, 1, O1 + i0 + (int64_t)i1 * sn,
+                         sn, 1, ph == 3);
+                }
+              wo += (int64_t)M * N;
+            }
+        }
+        dm.wsz = std::max(dm.wsz, wo);
+        dm.inv_phases.push_back({first, (int64_t)tiles.size() - first});
+      }
+    const int64_t first = (int64_t)tiles.size();
     for (int32_t i = 0; i < nf; ++i) {
       const FrontInfo &F = sy.fronts[i];
-      for (int kind = 0; kind < 2; ++kind) {
-        const int32_t M = kind ? F.s : F.u, N = kind ? F.u : F.s;
-        for (int32_t r0 = 0; r0 < M; r0 += TL)
-          for (int32_t c0 = 0; c0 < N; c0 += TL) {
-            tasks.push_back(i); tasks.push_back(kind); tasks.push_back(r0); tasks.push_back(c0);
-          }
-      }
+      const int32_t f = F.f, sn = F.s, u = F.u;
+      const int64_t O0 = io[i], O1 = io[i] + (int64_t)f * sn;
+      for (int32_t r = 0; r < u; r += TL)  // Fwd[s + i, j] = -sum_{k >= j} L21[i, k] Linv[k, j]
+        for (int32_t c = 0; c < sn; c += TL)
+          tile(u, sn, r, c, c, sn, 0, F.off + sn, f, 1, O0, f, 1, O0 + sn, f, 1);
+      for (int32_t r = 0; r < sn; r += TL)  // Bwd[i, s + c] = -sum_{k >= i} Uinv[i, k] U12[k, c]
+        for (int32_t c = 0; c < u; c += TL)
+          tile(sn, u, r, c, r, sn, 1, O1, sn, 0, F.off + (int64_t)sn * f, f, 1, O1 + (int64_t)sn * sn, sn, 1);
     }
-    dm.wz_cnt = ((int64_t)tasks.size() - dm.wz_off) / 4;
+    dm.inv_phases.push_back({first, (int64_t)tiles.size() - first});
+    dm.wsz = std::max<int64_t>(dm.wsz, 1);
+    dm.inv_tiles.upload(tiles, s);
   }
   dm.tasks.upload(tasks, s);
   if (d2) launch_elem_integrals(dm, s);
@@ -443,7 +501,7 @@ void lu_solve_host(Ctx *c, DevMesh &dm, int nb, const double *mat1, int nrhs, co
   int32_t *sig = c->buf<int32_t>("sig", (size_t)nb * sy.npiv);
   int32_t *gx = c->buf<int32_t>("gx", (size_t)nb * sy.npiv * 4);
   zd *inv = c->buf<zd>("inv", (size_t)nb * dm.isz);
-  lu_factor(dm, nb, m1, pool, piv, pfl, sig, gx, inv, c->stream);
+  lu_factor(dm, nb, m1, pool, piv, pfl, sig, gx, inv, c->buf<zd>("inv_w", (size_t)nb * dm.wsz), c->stream);
   zd *bo = c->buf<zd>("lu_b", (size_t)nb * nrhs * n);
   zd *bn = c->buf<zd>("lu_bn", (size_t)nb * nrhs * n);
   zd *yn = c->buf<zd>("lu_y", (size_t)nb * nrhs * n);
@@ -1309,7 +1367,7 @@ static SolveOut factor_solve_sort(Ctx *c, DevMesh &dm, const ModesArgs &a, int n
   int32_t *sig = c->buf<int32_t>("sig", (size_t)nb * sy.npiv);
   int32_t *gx = c->buf<int32_t>("gx", (size_t)nb * sy.npiv * 4);
   zd *inv = c->buf<zd>("inv", (size_t)nb * dm.isz);
-  lu_factor(dm, nb, m1, pool, piv, o.pflag, sig, gx, inv, s);
+  lu_factor(dm, nb, m1, pool, piv, o.pflag, sig, gx, inv, c->buf<zd>("inv_w", (size_t)nb * dm.wsz), s);
   float2 *inv32 = nullptr;
   if (a.precision == 1) {
     inv32 = c->buf<float2>("inv32", (size_t)nb * dm.isz);

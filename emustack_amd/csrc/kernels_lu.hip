@@ -738,7 +738,7 @@ static void launch_panel(const int32_t *tasks, unsigned cnt, int nb, int k0, int
 }
 
 void lu_factor(DevMesh &dm, int nb, const zd *mat1, zd *pool, int32_t *piv, int32_t *pflag, int32_t *sig,
-               int32_t *gx, zd *inv, hipStream_t s) {
+               int32_t *gx, zd *inv, zd *wt, hipStream_t s) {
   const Symbolic &sy = dm.host.sym;
   const int64_t psz = sy.pool;
   FrontArrays A = fa(dm);
@@ -768,7 +768,7 @@ void lu_factor(DevMesh &dm, int nb, const zd *mat1, zd *pool, int32_t *piv, int3
                            dm.tasks.p + L.ea_off[sl], A, pool, psz);
     EMU_LAUNCH_CHECK();
   }
-  lu_invert(dm, nb, pool, inv, s);
+  lu_invert(dm, nb, pool, inv, wt, s);
   const int nf = (int)sy.fronts.size();
   if (nf)
     hipLaunchKernelGGL(k_gather_index, dim3((unsigned)nf, nb), dim3(64), 0, s, A, sig, sy.npiv,
@@ -788,198 +788,228 @@ void lu_factor(DevMesh &dm, int nb, const zd *mat1, zd *pool, int32_t *piv, int3
 // column-sequential substitution inside one workgroup.  P is the front's
 // row-pivot permutation, applied as a gather (the gx records).
 
-constexpr int TB = 32;  // triangular block of the inversion
+// The triangular inverses are formed by doubling: k_tri_diag inverts the
+// 64 x 64 diagonal blocks, then for h = 64, 128, ... each pair of inverted
+// diagonal blocks A (h) and C gets its off-diagonal block B' = -C^-1 (B A^-1)
+// (lower) or -A^-1 (B C^-1) (upper) as two products of 64 x 64 tiles
+// (k_inv_gemm), all pairs of all fronts in one launch each, and two more that
+// correct it by its residual: U11 is ill-conditioned (1e6 on the case-1 cell)
+// and the plain products would leave solve residuals up to ten times those of
+// a substitution (8e-9 against 1e-9; 1e-9 with the correction).  The two
+// off-diagonal blocks of the inverted form follow as tiles of the same kernel.
+// Column-block substitution (one workgroup per 32 columns walking down the
+// front) was a serial chain of s / 32 products and 32-step solves.  Both parts
+// per factorisation: 8,000-triangle mesh, 2 / 8 instances, 6.4 / 15.5 ms, now
+// 2.9 / 8.8 ms; 64 dense matrices of order 98 and 200 (mean) 403 us, now 194 us.
+typedef double v4d __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ zd shfl_z(zd v, int lane) {
-  return zmk(__shfl(v.x, lane, 64), __shfl(v.y, lane, 64));
+// acc += A B on 16 x 16 x 4 complex blocks: a = A[i][k] in lane i + 16 k,
+// x = B[k][j] in lane j + 16 k; result D[i][j] in lane j + 16 (i mod 4),
+// register i / 4.
+__device__ __forceinline__ void mfma_z(v4d &re, v4d &im, zd a, zd x) {
+  re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x.x, re, 0, 0, 0);
+  im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, x.y, im, 0, 0, 0);
+  re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, x.y, re, 0, 0, 0);
+  im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, x.x, im, 0, 0, 0);
 }
 
-// One workgroup per (front, column block J, kind, instance): column block J
-// of L11^{-1} (kind 0, unit lower) or U11^{-1} (kind 1, upper) by blocked
-// substitution against identity columns.  Column blocks are independent.
-__global__ __launch_bounds__(256) void k_triinv(const int32_t *__restrict__ tasks, FrontArrays A,
-                                                const zd *__restrict__ pool, int64_t psz, zd *__restrict__ inv,
-                                                int64_t isz) {
+// Eight steps of the substitution of k_tri_diag, from row j0 of the block at
+// o: the ring a holds rows j0 .. j0 + 7, b the eight rows after them (FIRST).
+template <bool FIRST>
+__device__ __forceinline__ void tri_half(const zd (*__restrict__ T)[65], const zd *__restrict__ dinv, int o, int j0,
+                                         zd (&a)[8], zd (&b)[8]) {
+#pragma unroll 1
+  for (int jj = 0; jj < 8; ++jj) {
+    const int j = j0 + jj;
+    const zd l = zmul(a[0], dinv[j]);
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      const zd u = i < 8 - jj ? T[min(j + i, 63)][j] : zmk(0, 0);
+      a[i - 1] = zfms(u, l, a[i]);
+    }
+    a[7] = l;
+    if (FIRST)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) b[i] = zfms(T[o + 8 + i][j], l, b[i]);
+  }
+}
+
+// One workgroup per (front, 64-row diagonal block J, kind, instance): the
+// block's inverse, zeros of the other triangle included (the solves and the
+// products below read nothing outside the diagonal 64-blocks and the
+// triangle).  kind 0: L11 (unit lower); kind 1: U11, handled as a lower
+// triangle by reversing rows and columns.  The block sits in LDS, padded with
+// the identity, and X = T^-1 replaces it 16 rows at a time: the product of
+// the rows with the finished rows of X on the matrix cores, then a substitution
+// with the 16 x 16 diagonal block, one lane per column.  (Multiplying by an
+// inverted diagonal block instead would be shorter, but U11's blocks are
+// ill-conditioned, 1e6 on the case-1 cell, and its rounding then grows to ten
+// times that of the substitution.)
+__global__ __launch_bounds__(256) void k_tri_diag(const int32_t *__restrict__ tasks, FrontArrays A,
+                                                  const zd *__restrict__ pool, int64_t psz, zd *__restrict__ inv,
+                                                  int64_t isz) {
+  constexpr int D = 64, E = 16;
   const int t = tasks[3 * blockIdx.x], J = tasks[3 * blockIdx.x + 1], kind = tasks[3 * blockIdx.x + 2];
   const int b = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int s = A.s[t], f = A.f[t];
-  const zd *F = pool + b * psz + A.off[t];
-  zd *O = inv + b * isz + A.ioff[t] + (kind ? (int64_t)f * s : 0);
+  const int j0 = J * D, w = min(D, s - j0);
+  const zd *F = pool + b * psz + A.off[t] + j0 + (int64_t)j0 * f;
   const int64_t ldo = kind ? s : f;
-  const int nbk = (s + TB - 1) / TB;
-  const int j0 = J * TB, wj = min(TB, s - j0);
-  __shared__ zd Ts[TB][TB + 1];
-  __shared__ zd Xs[TB][TB + 1];
-  const int r = tid & 31, cg = tid >> 5;  // rows r, columns cg + 8m
-  // structural zeros of this column block
-  {
-    const int z0 = kind ? j0 + wj : 0, z1 = kind ? s : j0;
-    for (int idx = tid; idx < (z1 - z0) * wj; idx += 256) {
-      int i = z0 + idx % (z1 - z0), c = idx / (z1 - z0);
-      O[i + (int64_t)(j0 + c) * ldo] = zmk(0, 0);
-    }
+  zd *O = inv + b * isz + A.ioff[t] + (kind ? (int64_t)f * s : 0) + j0 + j0 * ldo;
+  __shared__ zd T[D][D + 1];
+  __shared__ zd dinv[D];
+  for (int idx = tid; idx < D * D; idx += 256) {
+    const int i = idx % D, j = idx / D;
+    const int fi = kind ? w - 1 - i : i, fj = kind ? w - 1 - j : j;
+    const zd v = F[min(max(fi, 0), w - 1) + (int64_t)min(max(fj, 0), w - 1) * f];
+    T[i][j] = (i < w && j <= i) ? v : zmk(0, 0);
   }
-  const int Ib = J, Ie = kind ? -1 : nbk, dI = kind ? -1 : 1;
-  for (int I = Ib; I != Ie; I += dI) {
-    const int i0 = I * TB, wi = min(TB, s - i0);
-    zd acc[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int c = cg + 8 * m;
-      acc[m] = (I == J && r == c) ? zmk(1, 0) : zmk(0, 0);
-    }
-    const int Kb = kind ? I + 1 : J, Ke = kind ? J + 1 : I;
-    for (int K = Kb; K < Ke; ++K) {
-      const int k0 = K * TB, wk = min(TB, s - k0);
-#pragma unroll
-      for (int u = 0; u < TB * TB / 256; ++u) {
-        const int idx = tid + 256 * u, i = idx % TB, kk = idx / TB;
-        const zd a = F[(i0 + min(i, wi - 1)) + (int64_t)(k0 + min(kk, wk - 1)) * f];
-        const zd x = O[(k0 + min(i, wk - 1)) + (int64_t)(j0 + min(kk, wj - 1)) * ldo];
-        Ts[i][kk] = (i < wi && kk < wk) ? a : zmk(0, 0);
-        Xs[i][kk] = (i < wk && kk < wj) ? x : zmk(0, 0);
-      }
-      __syncthreads();
-#pragma unroll 4
-      for (int kk = 0; kk < TB; ++kk) {
-        const zd a = Ts[r][kk];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) acc[m] = zfms(a, Xs[kk][cg + 8 * m], acc[m]);
-      }
-      __syncthreads();
-    }
-#pragma unroll
-    for (int u = 0; u < TB * TB / 256; ++u) {
-      const int idx = tid + 256 * u, i = idx % TB, j = idx / TB;
-      const zd a = F[(i0 + min(i, wi - 1)) + (int64_t)(i0 + min(j, wi - 1)) * f];
-      Ts[i][j] = (i < wi && j < wi) ? a : zmk(0, 0);
-    }
-#pragma unroll
-    for (int m = 0; m < 4; ++m) Xs[r][cg + 8 * m] = acc[m];
+  __syncthreads();
+  if (tid < D) dinv[tid] = kind && tid < w ? zdiv(zmk(1, 0), T[tid][tid]) : zmk(1, 0);
+  __syncthreads();
+  const int fi = lane & 15, fk = lane >> 4;
+#pragma unroll 1
+  for (int o = 0; o < w; o += E) {
+    // rows o .. o + 15 of -T X over the finished rows of X: wave v the columns
+    // 16 v .. 16 v + 15, written over the entries of T that they come from
+    const int cv = E * wave;
+    v4d re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+    if (cv < o)
+      for (int k = cv; k < o; k += 4) mfma_z(re, im, T[o + fi][k + fk], T[k + fk][cv + fi]);
     __syncthreads();
-    for (int c = wave; c < wj; c += 4) {
-      zd v = lane < wi ? Xs[lane][c] : zmk(0, 0);
-      if (kind == 0) {
-        for (int k = 0; k < wi - 1; ++k) {
-          const zd xk = shfl_z(v, k);
-          if (lane > k && lane < wi) v = zfms(Ts[lane][k], xk, v);
+    if (cv < o)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) T[o + fk + 4 * r][cv + fi] = zmk(-re[r], -im[r]);
+    __syncthreads();
+    if (wave == 0) {  // lane = column: substitution with the 16 x 16 diagonal block
+      constexpr int H = E / 2;
+      zd xa[H], xb[H];
+#pragma unroll
+      for (int i = 0; i < H; ++i) {
+        const zd va = T[o + i][lane], vb = T[o + H + i][lane];
+        xa[i] = lane < o ? va : zmk(lane == o + i ? 1.0 : 0.0, 0.0);
+        xb[i] = lane < o ? vb : zmk(lane == o + H + i ? 1.0 : 0.0, 0.0);
+      }
+      tri_half<true>(T, dinv, o, o, xa, xb);
+      tri_half<false>(T, dinv, o, o + H, xb, xa);
+      wave_sync();
+      if (lane < o + E)
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+          T[o + i][lane] = xa[i];
+          T[o + H + i][lane] = xb[i];
         }
-      } else {
-        for (int k = wi - 1; k >= 0; --k) {
-          const zd xk = zdiv(shfl_z(v, k), Ts[k][k]);
-          if (lane == k) v = xk;
-          else if (lane < k) v = zfms(Ts[lane][k], xk, v);
-        }
-      }
-      if (lane < wi) Xs[lane][c] = v;
     }
     __syncthreads();
-    for (int idx = tid; idx < wi * wj; idx += 256) {
-      int i = idx % wi, c = idx / wi;
-      O[(i0 + i) + (int64_t)(j0 + c) * ldo] = Xs[i][c];
-    }
-    __syncthreads();
+  }
+  for (int idx = tid; idx < w * w; idx += 256) {
+    const int i = idx % w, j = idx / w;
+    const int ti = kind ? w - 1 - i : i, tj = kind ? w - 1 - j : j;
+    O[i + j * ldo] = ti >= tj ? T[ti][tj] : zmk(0, 0);
   }
 }
 
-// Off-diagonal blocks of the inverted form (64 x 64 output tiles):
-//   kind 0:  Fwd[s+i, j] = -sum_{k>=j} L21[i,k] Linv[k,j]
-//   kind 1:  Bwd[i, s+c] = -sum_{k>=i} Uinv[i,k] U12[k,c]
-__global__ __launch_bounds__(256) void k_wz(const int32_t *__restrict__ tasks, FrontArrays A,
-                                            const zd *__restrict__ pool, int64_t psz, zd *__restrict__ inv,
-                                            int64_t isz) {
-  const int t = tasks[4 * blockIdx.x], kind = tasks[4 * blockIdx.x + 1];
-  const int r0 = tasks[4 * blockIdx.x + 2], c0 = tasks[4 * blockIdx.x + 3];
+// One 64 x 64 tile C = A B, -A B, C + A B or C - A B of the inversion (InvTile:
+// base arrays, offsets, leading dimensions, extents).  As k_zgemm_nn: 16-deep K rounds in
+// LDS, the next round fetched from clamped addresses meanwhile, wave w owns
+// columns 16 w .. 16 w + 15; 16-column blocks and the lower
+// half beyond the tile's extents are skipped
+// (most fronts are smaller than a tile).  FLOP-bound: a full tile takes 64 x 64
+// x 16 x 8 flops / 128 per clock = 4,096 clocks a round.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) void k_inv_gemm(const InvTile *__restrict__ tiles, const zd *__restrict__ pool,
+                                                  int64_t psz, zd *__restrict__ inv, int64_t isz,
+                                                  zd *__restrict__ wt, int64_t wsz) {
+  const InvTile R = tiles[blockIdx.x];
   const int b = blockIdx.y;
-  const int tid = threadIdx.x;
-  const int s = A.s[t], f = A.f[t];
-  const zd *F = pool + b * psz + A.off[t];
-  zd *Ofw = inv + b * isz + A.ioff[t];
-  zd *Obw = Ofw + (int64_t)f * s;
-  const int M = kind ? s : A.u[t], N = kind ? A.u[t] : s;
-  const int kbeg = kind ? r0 : c0;
-  // K staged in rounds of GK (32 KB of LDS, four workgroups per CU); the next
-  // round's operands are fetched into registers while this one is used, from
-  // clamped addresses, and masked when stored to LDS (a select right after
-  // the load would wait for it at once)
-  __shared__ zd As[GK][TILE];
-  __shared__ zd Bs[GK][TILE];
-  const int tx = tid % 16, ty = tid / 16;  // rows tx + 16 i, columns ty + 16 j
-  zd acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = zmk(0, 0);
-  constexpr int NL = GK * TILE / 256;
-  zd ra[NL], rb[NL];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  zd *const base1 = inv + b * isz, *const base2 = wt + b * wsz;
+  const zd *Ab = (R.abase == 0 ? pool + b * psz : R.abase == 1 ? (const zd *)base1 : base2) + R.aoff;
+  const zd *Bb = (R.bbase == 0 ? pool + b * psz : R.bbase == 1 ? (const zd *)base1 : base2) + R.boff;
+  zd *Cb = (R.cbase == 1 ? base1 : base2) + R.coff;
+  __shared__ zd As[GK][TILE + 1];
+  __shared__ zd Bs[GK][TILE + 1];
+  const int am = tid & 63, ak = tid >> 6;  // A: row am, K columns ak + 4 i
+  const int bk = tid & 15, bn = tid >> 4;  // B: K row bk, columns bn + 16 i
+  zd ra[4], rb[4];
   auto fetch = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < NL; ++u) {
-      const int idx = tid + 256 * u, i = idx % TILE, kk = idx / TILE;
-      const int rc = min(r0 + i, M - 1), kc = min(k0 + kk, s - 1);
-      ra[u] = kind ? Obw[rc + (int64_t)kc * s] : F[(s + rc) + (int64_t)kc * f];
-    }
+    for (int i = 0; i < 4; ++i) ra[i] = Ab[min(am, R.M - 1) + (int64_t)min(k0 + ak + 4 * i, R.K - 1) * R.lda];
+    const int kb = min(k0 + bk, R.K - 1);
 #pragma unroll
-    for (int u = 0; u < NL; ++u) {
-      const int idx = tid + 256 * u, kk = idx % GK, jj = idx / GK;
-      const int ccc = min(c0 + jj, N - 1), kc = min(k0 + kk, s - 1);
-      rb[u] = kind ? F[kc + (int64_t)(s + ccc) * f] : Ofw[kc + (int64_t)ccc * f];
-    }
+    for (int i = 0; i < 4; ++i) rb[i] = Bb[kb + (int64_t)min(bn + 16 * i, R.N - 1) * R.ldb];
   };
-  if (kbeg < s) fetch(kbeg);
-  for (int k0 = kbeg; k0 < s; k0 += GK) {
+  v4d re[4], im[4];
 #pragma unroll
-    for (int u = 0; u < NL; ++u) {
-      const int idx = tid + 256 * u, i = idx % TILE, kk = idx / TILE;
-      As[kk][i] = (r0 + i < M && k0 + kk < s) ? ra[u] : zmk(0, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < NL; ++u) {
-      const int idx = tid + 256 * u, kk = idx % GK, jj = idx / GK;
-      Bs[kk][jj] = (c0 + jj < N && k0 + kk < s) ? rb[u] : zmk(0, 0);
-    }
-    __syncthreads();
-    if (k0 + GK < s) fetch(k0 + GK);
-#pragma unroll 2
-    for (int kk = 0; kk < GK; ++kk) {
-      zd a[4], bb[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][tx + 16 * i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bb[j] = Bs[kk][ty + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = zfma(a[i], bb[j], acc[i][j]);
-    }
-    __syncthreads();
+  for (int t = 0; t < 4; ++t) {
+    re[t] = (v4d){0, 0, 0, 0};
+    im[t] = (v4d){0, 0, 0, 0};
   }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int cc = c0 + ty + 16 * j;
+  const int fi = lane & 15, fk = lane >> 4;
+  fetch(0);
+  for (int k0 = 0; k0 < R.K; k0 += GK) {
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int rr = r0 + tx + 16 * i;
-      if (rr < M && cc < N) {
-        const zd v = zmk(-acc[i][j].x, -acc[i][j].y);
-        if (kind) Obw[rr + (int64_t)(s + cc) * s] = v;
-        else Ofw[(s + rr) + (int64_t)cc * f] = v;
+      const int kk = ak + 4 * i, d = k0 + kk - am - R.doff;  // columns right of the diagonal
+      bool ok = k0 + kk < R.K && am < R.M;
+      if (R.tri == 1) ok = ok && d < 0;
+      if (R.tri == 2) ok = ok && d >= 0;
+      As[kk][am] = ok ? ra[i] : zmk(R.tri == 1 && d == 0 ? 1.0 : 0.0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) Bs[bk][bn + 16 * i] = (k0 + bk < R.K && bn + 16 * i < R.N) ? rb[i] : zmk(0, 0);
+    __syncthreads();
+    if (k0 + GK < R.K) fetch(k0 + GK);
+    if (16 * wv < R.N) {
+      if (R.M > 32) {
+#pragma unroll
+        for (int ks = 0; ks < GK / 4; ++ks) {
+          const int kk = ks * 4 + fk;
+          const zd xb = Bs[kk][16 * wv + fi];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) mfma_z(re[t], im[t], As[kk][16 * t + fi], xb);
+        }
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < GK / 4; ++ks) {
+          const int kk = ks * 4 + fk;
+          const zd xb = Bs[kk][16 * wv + fi];
+#pragma unroll
+          for (int t = 0; t < 2; ++t) mfma_z(re[t], im[t], As[kk][16 * t + fi], xb);
+        }
       }
     }
   }
+  const int n = 16 * wv + fi;
+  if (n >= R.N) return;
+  Cb += (int64_t)n * R.ldc;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = 16 * t + fk + 4 * r;
+      if (m < R.M) {
+        zd v = R.neg ? zmk(-re[t][r], -im[t][r]) : zmk(re[t][r], im[t][r]);
+        if (R.acc) v = zadd(Cb[m], v);
+        Cb[m] = v;
+      }
+    }
 }
 
-void lu_invert(DevMesh &dm, int nb, const zd *pool, zd *inv, hipStream_t s) {
+void lu_invert(DevMesh &dm, int nb, const zd *pool, zd *inv, zd *wt, hipStream_t s) {
   const Symbolic &sy = dm.host.sym;
   FrontArrays A = fa(dm);
   if (dm.tri_cnt)
-    hipLaunchKernelGGL(k_triinv, dim3((unsigned)dm.tri_cnt, nb), dim3(256), 0, s, dm.tasks.p + dm.tri_off, A, pool,
+    hipLaunchKernelGGL(k_tri_diag, dim3((unsigned)dm.tri_cnt, nb), dim3(256), 0, s, dm.tasks.p + dm.tri_off, A, pool,
                        sy.pool, inv, dm.isz);
   EMU_LAUNCH_CHECK();
-  if (dm.wz_cnt)
-    hipLaunchKernelGGL(k_wz, dim3((unsigned)dm.wz_cnt, nb), dim3(256), 0, s, dm.tasks.p + dm.wz_off, A, pool,
-                       sy.pool, inv, dm.isz);
+  for (const auto &r : dm.inv_phases)
+    if (r.second > 0)
+      hipLaunchKernelGGL(k_inv_gemm, dim3((unsigned)r.second, nb), dim3(256), 0, s, dm.inv_tiles.p + r.first, pool,
+                         sy.pool, inv, dm.isz, wt, dm.wsz);
   EMU_LAUNCH_CHECK();
 }
 
