@@ -59,9 +59,9 @@ struct KTime {
 // Live kernel timing (enabled by emu_profile).  A "sweep" is one solve or one
 // Gram-Schmidt pass; every `every`-th sweep is recorded.  Classes: 0 forward
 // solve (k_fwd), 1 backward solve (k_bwd), 2 Gram-Schmidt projection
-// (k_atb_mfma16; k_atb_tall below 8-column blocks), 3 Gram-Schmidt update
-// (k_combine; k_sub_vh_blk below 8-column blocks), 4 sparse M product of the
-// Krylov block (k_spmm_il; k_spmm below 8 columns); per class: dispatches,
+// (k_atb_mfma16; k_atb_tall for single vectors), 3 Gram-Schmidt update
+// (k_combine; k_sub_vh_blk for single vectors), 4 sparse M product of the
+// Krylov block (k_spmm_il; k_spmm for single vectors); per class: dispatches,
 // milliseconds, algorithmic bytes.
 struct Profiler {
   bool on = false;
@@ -298,21 +298,21 @@ void launch_permute_vec(DevMesh &dm, int nb, int ncol, const zd *src, zd *dst, b
 
 // ---------------- dense / vector kernels (kernels_krylov.hip) ----------------
 // y[b][r] = sum_k A[b][r][k] x[b][col k] for CSR (n x n), ncol columns
-// M times one 8-column block X (column-major, ld n) through the
-// row-interleaved scratch xi (nb x 8 n): y column-major (ld n).  xi_ready:
+// M times one block X of bq = 2, 4 or 8 columns (column-major, ld n) through
+// the row-interleaved scratch xi (nb x bq n): y column-major (ld n).  xi_ready:
 // xi already holds X's interleaved copy (written by launch_trmm_right)
-void launch_spmm8_il(int nb, int64_t n, const int64_t *rp, const int32_t *ci, const zd *vals, int64_t vstride,
-                     const zd *x, int64_t xstride, zd *xi, zd *y, int64_t ystride, hipStream_t s, KTime kt = {},
-                     bool xi_ready = false);
+void launch_spmm_il(int nb, int64_t n, int bq, const int64_t *rp, const int32_t *ci, const zd *vals, int64_t vstride,
+                    const zd *x, int64_t xstride, zd *xi, zd *y, int64_t ystride, hipStream_t s, KTime kt = {},
+                    bool xi_ready = false);
 // xi (optional, nb x n x ncol): scratch for the row-major copy that the
 // many-column form (ncol > 8) works from
 void launch_spmm(int nb, int64_t n, int ncol, const int64_t *rp, const int32_t *ci, const zd *vals,
                  int64_t vstride, const zd *x, int64_t xstride, zd *y, int64_t ystride,
                  hipStream_t s, KTime kt = {}, zd *xi = nullptr);
 // C[b] (M x N, ldc) = op(A[b])^T B[b] with K rows; op = conj if conjA, split
-// over K (partial products per K chunk in scratch, then a reduction).  N in
-// {1, 2, 4, 8, 16}: the tall-skinny kernel (the one kt times); 8 x 8 Gram
-// matrices of a block: a dedicated kernel; other N: 64 x 64 MFMA output tiles.
+// over K (partial products per K chunk in scratch, then a reduction).  N = 1:
+// the single-column kernel (the one kt times); other N: 64 x 64 MFMA output
+// tiles.
 void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64_t sA,
                 const zd *B, int64_t ldb, int64_t sB, zd *C, int64_t ldc, int64_t sC,
                 bool conjA, zd *scratch, size_t scratch_elems, hipStream_t s, KTime kt = {});
@@ -336,22 +336,38 @@ void launch_swap_i32(int64_t n, int32_t *a, int32_t *b, hipStream_t s);
 // block Gram-Schmidt: W[:, :bq] -= V[:, :k] H[:k, :bq]
 void launch_sub_vh_blk(int nb, int64_t n, int k, int bq, const zd *V, int64_t ldv, int64_t sV, const zd *H,
                        int64_t ldh, int64_t sH, zd *W, int64_t ldw, int64_t sW, hipStream_t s, KTime kt = {});
-// Delayed block Gram-Schmidt (block size 8): W (n x nq, in place) = W L - V[:, :k] E
-// (E row-major, k x nq per instance)
-void launch_combine(int nb, int64_t n, int k, int nq, const zd *V, int64_t ldv, int64_t sV, const zd *E,
-                    int64_t sE, const zd *L, zd *W, int64_t ldw, int64_t sW, hipStream_t s, KTime kt = {});
-// ... and the coefficients of one step (fin: reorthogonalise the last block only)
-void launch_dcgs_coef(int nb, bool fin, int j, int c0, const zd *P, int64_t ldp, int64_t sP, const zd *A0,
-                      int64_t lda, int64_t sA, zd *H, int64_t ldh, int64_t sH, zd *E, int64_t sE, zd *L, int32_t *bad,
-                      hipStream_t s);
-// Cholesky-QR of a bq-column block: G = R^H R, Rinv = R^-1, Racc = R * Rprev
-void launch_cholqr(int nb, int bq, const zd *G, zd *Rinv, const zd *Rprev, zd *Racc, int32_t *bad,
-                   hipStream_t s);
-// O = W * Rinv (bq x bq upper triangular), in place allowed; for bq = 8 and
-// xi given, O is also written row-interleaved to xi (nb x 8 n, the layout
-// launch_spmm8_il reads)
-void launch_trmm_right(int nb, int64_t n, int bq, const zd *W, int64_t ldw, int64_t sW, const zd *Ri, zd *O,
-                       int64_t ldo, int64_t sO, hipStream_t s, zd *xi = nullptr);
+// Delayed block Gram-Schmidt (block size bq = 2, 4 or 8).  The projection
+// C[b] (M x N) = A[b]^H B[b], N = bq or 2 bq columns
+void launch_proj(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64_t sA, const zd *B, int64_t ldb,
+                 int64_t sB, zd *C, int64_t ldc, int64_t sC, zd *scratch, size_t scratch_elems, hipStream_t s,
+                 KTime kt = {});
+// ... the coefficients of one step (fin: reorthogonalise the last block only);
+// part: dcgs_part_elems entries per instance.  Row block j of H is left in
+// Hrow (bq x j per instance) for launch_cholqr (fin: stored)
+int64_t dcgs_part_elems(int bq, int m);
+void launch_dcgs(int nb, int bq, bool fin, int j, int c0, const zd *P, int64_t ldp, int64_t sP, zd *A0, int64_t lda,
+                 int64_t sA, zd *part, zd *H, int64_t ldh, int64_t sH, zd *E, int64_t sE, zd *L, zd *Hrow, int64_t sR,
+                 int32_t *bad, hipStream_t s);
+// ... and the update W (n x nq, in place) = W L - V[:, :k] E (E row-major, k x
+// nq per instance).  gpart (optional): partial Gram matrices of the last nq / 2
+// columns, one per row block; returns their number, 0 if they were not formed
+int64_t launch_combine(int nb, int64_t n, int k, int nq, const zd *V, int64_t ldv, int64_t sV, const zd *E,
+                       int64_t sE, const zd *L, zd *W, int64_t ldw, int64_t sW, zd *gpart, hipStream_t s, KTime kt = {});
+// Gram matrix of a block in partial sums per row block (returns their number;
+// gpart holds at most gram_blocks(n) of them per instance)
+inline int64_t gram_blocks(int64_t n) { return (n + 63) / 64; }
+int64_t launch_gram(int nb, int64_t n, int bq, const zd *W, int64_t ldw, int64_t sW, zd *gpart, hipStream_t s);
+// Cholesky-QR of a block from those: G = R^H R, Rinv = R^-1, Racc = R * Rprev;
+// with H: Racc to the subdiagonal block of column block j, Hrow to columns
+// [c0, j) of row block j
+void launch_cholqr(int nb, int bq, int64_t nchunk, const zd *gpart, zd *Rinv, const zd *Rprev, zd *Racc, int32_t *bad,
+                   hipStream_t s, int j = 0, int c0 = 0, const zd *Hrow = nullptr, int64_t sR = 0, zd *H = nullptr,
+                   int64_t ldh = 0, int64_t sH = 0);
+// O = W * Rinv (bq x bq upper triangular), in place allowed; with xi, O is
+// also written row-interleaved to xi (nb x bq n, the layout launch_spmm_il
+// reads); with gpart, its partial Gram matrices (returns the number of row blocks)
+int64_t launch_trmm_right(int nb, int64_t n, int bq, const zd *W, int64_t ldw, int64_t sW, const zd *Ri, zd *O,
+                          int64_t ldo, int64_t sO, hipStream_t s, zd *xi = nullptr, zd *gpart = nullptr);
 void launch_block_copy(int nb, int rows, int cols, const zd *S, int64_t lds, int64_t sS, zd *D, int64_t ldd,
                        int64_t sD, bool add, hipStream_t s);
 void launch_fill(zd *p, int64_t n, zd v, hipStream_t s);

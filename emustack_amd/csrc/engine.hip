@@ -523,8 +523,9 @@ void lu_solve_host(Ctx *c, DevMesh &dm, int nb, const double *mat1, int nrhs, co
 // Block Krylov-Schur (block size bq) for the nev largest-|mu| eigenpairs of
 // OP = (K - shift M)^-1 M, the operator ARPACK iterates on in the reference
 // (valpr_umf_64.f:291-459, which = 'LM').  One block step applies OP to bq
-// vectors (one multi-RHS solve), orthogonalises them against the basis with
-// two block classical Gram-Schmidt passes and Cholesky-QR2 inside the block.
+// vectors (one multi-RHS solve), orthogonalises them against the basis
+// (delayed block Gram-Schmidt; two classical passes for single vectors) and
+// inside the block (Cholesky-QR2).
 // The projected (m x m) Schur problem is solved on the host with LAPACK.
 //
 // Relation after the expansion:  OP V[:, :m] = V[:, :m+bq] H[:m+bq, :m].
@@ -741,17 +742,30 @@ struct StageTimer {
   }
 };
 
-// orthonormalise V[:, j:j+bq] in place (Cholesky-QR2); R (bq x bq) of the
-// factorisation W = Q R is written to Rout[b] (device, bq x bq) when given;
-// xi (8-column blocks): also write the row-interleaved copy of the result
-static void block_cholqr2(Ctx *c, int nb, int64_t n, int bq, zd *W, int64_t sV, zd *G, zd *Ri, zd *R1, zd *Rout,
-                          int32_t *bad, zd *atbs, size_t atb_elems, hipStream_t s, zd *xi = nullptr) {
-  const int64_t sG = (int64_t)bq * bq;
-  launch_atb(nb, n, bq, bq, W, n, sV, W, n, sV, G, bq, sG, true, atbs, atb_elems, s);
-  launch_cholqr(nb, bq, G, Ri, nullptr, R1, bad, s);
-  launch_trmm_right(nb, n, bq, W, n, sV, Ri, W, n, sV, s);
-  launch_atb(nb, n, bq, bq, W, n, sV, W, n, sV, G, bq, sG, true, atbs, atb_elems, s);
-  launch_cholqr(nb, bq, G, Ri, R1, Rout, bad, s);
+// Destination of a block step's Cholesky-QR results in H (launch_cholqr).
+struct HDest {
+  int j = 0, c0 = 0;
+  const zd *Hrow = nullptr;
+  int64_t sR = 0;
+  zd *H = nullptr;
+  int64_t ld = 0, sH = 0;
+};
+
+// orthonormalise the block W (n x bq) in place (Cholesky-QR2); R of the
+// factorisation W = Q R is written to Rout[b] (device, bq x bq) and to H when
+// given; nchunk > 0: gpart already holds W's Gram partials (launch_combine);
+// xi: also write the row-interleaved copy of the result
+static void block_cholqr2(int nb, int64_t n, int bq, zd *W, int64_t sV, zd *gpart, int64_t nchunk, zd *Ri, zd *R1,
+                          zd *Rout, int32_t *bad, hipStream_t s, zd *xi = nullptr, const HDest &hd = {}) {
+  if (nchunk <= 0) nchunk = launch_gram(nb, n, bq, W, n, sV, gpart, s);
+  if (bq == 1) {  // one vector: a second normalisation would change its length by rounding only
+    launch_cholqr(nb, bq, nchunk, gpart, Ri, nullptr, Rout, bad, s, hd.j, hd.c0, hd.Hrow, hd.sR, hd.H, hd.ld, hd.sH);
+    launch_trmm_right(nb, n, bq, W, n, sV, Ri, W, n, sV, s);
+    return;
+  }
+  launch_cholqr(nb, bq, nchunk, gpart, Ri, nullptr, R1, bad, s);
+  nchunk = launch_trmm_right(nb, n, bq, W, n, sV, Ri, W, n, sV, s, nullptr, gpart);
+  launch_cholqr(nb, bq, nchunk, gpart, Ri, R1, Rout, bad, s, hd.j, hd.c0, hd.Hrow, hd.sR, hd.H, hd.ld, hd.sH);
   launch_trmm_right(nb, n, bq, W, n, sV, Ri, W, n, sV, s, xi);
 }
 
@@ -805,11 +819,12 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
   zd *V2 = c->buf<zd>("ks_V2", (size_t)nb * sV);
   zd *t1 = c->buf<zd>("ks_t1", (size_t)nb * bq * n);
   zd *ty = c->buf<zd>("ks_ty", (size_t)nb * bq * n);
-  zd *xil = bq == 8 ? c->buf<zd>("ks_xil", (size_t)nb * 8 * n) : nullptr;  // interleaved SpMM input
+  const bool delayed = bq > 1;  // delayed block Gram-Schmidt (2, 4 or 8 columns)
+  zd *xil = delayed ? c->buf<zd>("ks_xil", (size_t)nb * bq * n) : nullptr;  // interleaved SpMM input
   zd *tw = c->buf<zd>("ks_w", (size_t)nb * bq * solve_ws(dm));
   zd *Hd = c->buf<zd>("ks_H", (size_t)nb * sH);
   zd *H2 = c->buf<zd>("ks_H2", (size_t)nb * ld * bq);
-  zd *G = c->buf<zd>("ks_G", (size_t)nb * bq * bq);
+  zd *gpart = c->buf<zd>("ks_gpart", (size_t)nb * bq * bq * gram_blocks(n));
   zd *Ri = c->buf<zd>("ks_Ri", (size_t)nb * bq * bq);
   zd *R1 = c->buf<zd>("ks_R1", (size_t)nb * bq * bq);
   zd *Rf = c->buf<zd>("ks_Rf", (size_t)nb * bq * bq);
@@ -817,14 +832,15 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
   size_t atb_elems = (size_t)nb * (m + bq) * std::max(bq, 32) * 128;
   zd *atbs = c->buf<zd>("ks_atb", atb_elems);
   zd *Qd = c->buf<zd>("ks_Q", (size_t)nb * m * m);
-  // delayed block Gram-Schmidt (block size 8): projections and Gram matrix
+  // delayed block Gram-Schmidt: projections and Gram matrix
   // P = [V Z W]^H [Z W], A0 = H S, combination E, L
-  const bool delayed = bq == 8;
   const int64_t ldp = m + bq, sP = ldp * 2 * bq, sA0 = ldp * bq;
   zd *Pd = delayed ? c->buf<zd>("ks_P", (size_t)nb * sP) : nullptr;
   zd *A0d = delayed ? c->buf<zd>("ks_A0", (size_t)nb * sA0) : nullptr;
   zd *Ed = delayed ? c->buf<zd>("ks_E", (size_t)nb * sP) : nullptr;
   zd *Ld = delayed ? c->buf<zd>("ks_L", (size_t)nb * 4 * bq * bq) : nullptr;
+  zd *Cd = delayed ? c->buf<zd>("ks_cpart", (size_t)nb * dcgs_part_elems(bq, m)) : nullptr;
+  zd *Hr = delayed ? c->buf<zd>("ks_Hrow", (size_t)nb * sA0) : nullptr;
   EMU_HIP(hipMemsetAsync(bad, 0, sizeof(int32_t) * nb, s));
   // start block: deterministic pseudo-random, orthonormalised
   {
@@ -835,7 +851,7 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
     EMU_HIP(hipMemcpyAsync(t1, v0.data(), sizeof(zd) * v0.size(), hipMemcpyHostToDevice, s));
     EMU_HIP(hipStreamSynchronize(s));
     launch_copy(nb, bq * n, t1, bq * n, V, sV, s);
-    block_cholqr2(c, nb, n, bq, V, sV, G, Ri, R1, Rf, bad, atbs, atb_elems, s);
+    block_cholqr2(nb, n, bq, V, sV, gpart, 0, Ri, R1, Rf, bad, s);
   }
   launch_fill(Hd, (int64_t)nb * sH, zmk(0, 0), s);
   std::vector<KSState> st(nb);
@@ -893,9 +909,9 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
       zd *Wn = V + (int64_t)(j + bq) * n;  // next block slot
       if (pf) pf->start_sweep();
       const KTime kspmv = pf ? pf->time(4, nbd * (20.0 * nzd + 8.0 * (nd + 1) + 32.0 * nd * bq)) : KTime{};
-      if (bq == 8)
-        launch_spmm8_il(nact, n, dm.prow_ptr.p, dm.pcol_ind.p, mvals, dm.host.nnz, Xj, sV, xil, t1, (int64_t)bq * n,
-                        s, kspmv, xil_ready);
+      if (delayed)
+        launch_spmm_il(nact, n, bq, dm.prow_ptr.p, dm.pcol_ind.p, mvals, dm.host.nnz, Xj, sV, xil, t1, (int64_t)bq * n,
+                       s, kspmv, xil_ready);
       else
         launch_spmm(nact, n, bq, dm.prow_ptr.p, dm.pcol_ind.p, mvals, dm.host.nnz, Xj, sV, t1, (int64_t)bq * n, s,
                     kspmv);
@@ -910,15 +926,14 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
         const int c0 = j == k ? 0 : j - bq;
         // algorithmic bytes: one read of [V Z W] (j + 2 bq columns; [Z W] is
         // a slice of it); the combine reads V[:, :j] and [Z W] and writes [Z W]
-        launch_atb(nact, n, j + 2 * bq, 2 * bq, V, n, sV, Xj, n, sV, Pd, ldp, sP, true, atbs, atb_elems, s,
-                   pf ? pf->time(2, nbd * 16.0 * nd * (j + 2 * bq)) : KTime{});
-        if (j > 0) launch_gemm_nn(nact, j, bq, j, zmk(1, 0), Hd, ld, sH, Pd, ldp, sP, zmk(0, 0), A0d, ldp, sA0, s);
-        launch_dcgs_coef(nact, false, j, c0, Pd, ldp, sP, A0d, ldp, sA0, Hd, ld, sH, Ed, sP, Ld, bad, s);
-        launch_combine(nact, n, j, 2 * bq, V, n, sV, Ed, sP, Ld, Xj, n, sV, s,
-                       pf ? pf->time(3, nbd * 16.0 * nd * (j + 4 * bq)) : KTime{});
-        block_cholqr2(c, nact, n, bq, Wn, sV, G, Ri, R1, Rf, bad, atbs, atb_elems, s, bq == 8 ? xil : nullptr);
-        xil_ready = bq == 8;
-        launch_block_copy(nact, bq, bq, Rf, bq, (int64_t)bq * bq, Hd + (int64_t)j * ld + j + bq, ld, sH, false, s);
+        launch_proj(nact, n, j + 2 * bq, 2 * bq, V, n, sV, Xj, n, sV, Pd, ldp, sP, atbs, atb_elems, s,
+                    pf ? pf->time(2, nbd * 16.0 * nd * (j + 2 * bq)) : KTime{});
+        launch_dcgs(nact, bq, false, j, c0, Pd, ldp, sP, A0d, ldp, sA0, Cd, Hd, ld, sH, Ed, sP, Ld, Hr, sA0, bad, s);
+        const int64_t nch =
+            launch_combine(nact, n, j, 2 * bq, V, n, sV, Ed, sP, Ld, Xj, n, sV, gpart, s,
+                           pf ? pf->time(3, nbd * 16.0 * nd * (j + 4 * bq)) : KTime{});
+        block_cholqr2(nact, n, bq, Wn, sV, gpart, nch, Ri, R1, Rf, bad, s, xil, HDest{j, c0, Hr, sA0, Hd, ld, sH});
+        xil_ready = true;
         res.ops += (int64_t)nact * bq;
         res.steps += 1;
         continue;
@@ -933,17 +948,17 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
                           pf ? pf->time(3, nbd * 16.0 * nd * (j + 3 * bq)) : KTime{});
       }
       launch_block_copy(nact, j + bq, bq, H2, ld, (int64_t)ld * bq, Hd + (int64_t)j * ld, ld, sH, true, s);
-      block_cholqr2(c, nact, n, bq, Wn, sV, G, Ri, R1, Rf, bad, atbs, atb_elems, s);
-      launch_block_copy(nact, bq, bq, Rf, bq, (int64_t)bq * bq, Hd + (int64_t)j * ld + j + bq, ld, sH, false, s);
+      block_cholqr2(nact, n, bq, Wn, sV, gpart, 0, Ri, R1, Rf, bad, s, nullptr, HDest{j, j, nullptr, 0, Hd, ld, sH});
       res.ops += (int64_t)nact * bq;
       res.steps += 1;
     }
     if (delayed) {
       // reorthogonalise the last provisional block (the residual block of the
       // Krylov-Schur relation) and correct row block m of H
-      launch_atb(nact, n, m + bq, bq, V, n, sV, V + (int64_t)m * n, n, sV, Pd, ldp, sP, true, atbs, atb_elems, s);
-      launch_dcgs_coef(nact, true, m, m - bq, Pd, ldp, sP, nullptr, ldp, sA0, Hd, ld, sH, Ed, sP, Ld, bad, s);
-      launch_combine(nact, n, m, bq, V, n, sV, Ed, sP, Ld, V + (int64_t)m * n, n, sV, s);
+      launch_proj(nact, n, m + bq, bq, V, n, sV, V + (int64_t)m * n, n, sV, Pd, ldp, sP, atbs, atb_elems, s);
+      launch_dcgs(nact, bq, true, m, m - bq, Pd, ldp, sP, nullptr, ldp, sA0, Cd, Hd, ld, sH, Ed, sP, Ld, Hr, sA0, bad,
+                  s);
+      launch_combine(nact, n, m, bq, V, n, sV, Ed, sP, Ld, V + (int64_t)m * n, n, sV, nullptr, s);
     }
     tm.mark("krylov_expand");
     EMU_HIP(hipMemcpyAsync(Hh.data(), Hd, sizeof(zd) * (size_t)nact * sH, hipMemcpyDeviceToHost, s));

@@ -22,6 +22,7 @@ namespace emu {
 // x.
 constexpr int SM_C = 8;
 
+__device__ __forceinline__ zd shfl_z(zd v, int lane) { return zmk(__shfl(v.x, lane, 64), __shfl(v.y, lane, 64)); }
 __device__ __forceinline__ zd shfl_xor_z(zd v, int m) {
   return zmk(__shfl_xor(v.x, m, 64), __shfl_xor(v.y, m, 64));
 }
@@ -187,36 +188,41 @@ void launch_spmm(int nb, int64_t n, int ncol, const int64_t *rp, const int32_t *
 
 
 // ------------------------------------------- SpMM on a row-interleaved block
-// The Krylov loop multiplies M by one 8-column block per step.  Gathering
-// x[col] of eight columns stored n apart touches eight cache lines per
-// nonzero; with the block stored row-interleaved (xi[8 col + c]) the eight
-// values of a nonzero's column are one 128-byte line, read whole.  The block
-// is interleaved by one pass (k_interleave8, 2 x 16 n bytes per column
-// block) before the product.
-__global__ __launch_bounds__(256) void k_interleave8(int64_t n, const zd *__restrict__ X, int64_t sX,
-                                                     zd *__restrict__ xi, int64_t sI) {
+// The Krylov loop multiplies M by one B-column block per step.  Gathering
+// x[col] of B columns stored n apart touches B cache lines per nonzero; with
+// the block stored row-interleaved (xi[B col + c]) the B values of a nonzero's
+// column are one run (a 128-byte line at B = 8), read whole.  The block is
+// interleaved by k_trmm_right as it is written, or by one pass
+// (k_interleave, 2 x 16 n bytes per column block) before the product.
+template <int B>
+__global__ __launch_bounds__(256) void k_interleave(int64_t n, const zd *__restrict__ X, int64_t sX,
+                                                    zd *__restrict__ xi, int64_t sI) {
   const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const int b = blockIdx.y;
   if (r >= n) return;
   const zd *x = X + b * sX;
-  zd v[8];
+  zd v[B];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) v[c] = ld_stream(x + (int64_t)c * n + r);
-  zd *o = xi + b * sI + 8 * r;
+  for (int c = 0; c < B; ++c) v[c] = ld_stream(x + (int64_t)c * n + r);
+  zd *o = xi + b * sI + B * r;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) o[c] = v[c];
+  for (int c = 0; c < B; ++c) o[c] = v[c];
 }
 
+template <int B>
 __global__ __launch_bounds__(256) void k_spmm_il(int64_t n, const int64_t *__restrict__ rp,
                                                  const int32_t *__restrict__ ci, const zd *__restrict__ vals,
                                                  int64_t vstride, const zd *__restrict__ xi, int64_t xstride,
                                                  zd *__restrict__ y, int64_t ystride, int per) {
-  // Eight lanes share a row and lane c owns output column c.  Per step the
-  // group takes the row's next eight nonzeros (lane j loads value and column
-  // of nonzero j, coalesced), then for each of them lane c loads x[col][c]:
+  // Eight lanes share a row.  Per step the group takes the row's next eight
+  // nonzeros (lane j loads value and column of nonzero j, coalesced).  B = 8:
+  // lane c owns output column c and for each of the nonzeros loads x[col][c]:
   // the group reads one 128-byte line per nonzero, eight lines per wavefront
-  // load, and accumulates without a final cross-lane reduction.
-  const int lane8 = threadIdx.x & 7;
+  // load, and accumulates without a final cross-lane reduction.  B < 8: the
+  // lanes are 8 / B sets of B columns, each set takes every (8 / B)-th nonzero,
+  // and the sets' sums are added at the end.
+  constexpr int NS = 8 / B;
+  const int lane8 = threadIdx.x & 7, col8 = lane8 % B, set = lane8 / B;
   const int gbase = threadIdx.x & 63 & ~7;  // first lane of the group in the wavefront
   const int64_t blk = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
   const int64_t r = blk * 32 + (threadIdx.x >> 3);
@@ -233,32 +239,42 @@ __global__ __launch_bounds__(256) void k_spmm_il(int64_t n, const int64_t *__res
     const int col = ld_stream(ci + kc);
     if (!ok) a = zmk(0, 0);
     const int cnt = (int)min((int64_t)8, k1 - kb);
-    zd xv[8], av[8];
+    zd xv[B], av[B];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int cq = __shfl(col, gbase + q, 64);
-      av[q] = zmk(__shfl(a.x, gbase + q, 64), __shfl(a.y, gbase + q, 64));
-      xv[q] = xb[8 * (int64_t)cq + lane8];
+    for (int q = 0; q < B; ++q) {
+      const int src = gbase + NS * q + set;
+      const int cq = __shfl(col, src, 64);
+      av[q] = zmk(__shfl(a.x, src, 64), __shfl(a.y, src, 64));
+      xv[q] = xb[B * (int64_t)cq + col8];
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < 8; ++q)
-      if (q < cnt) acc = zfma(av[q], xv[q], acc);
+    for (int q = 0; q < B; ++q)
+      if (NS * q + set < cnt) acc = zfma(av[q], xv[q], acc);
   }
-  if (r < n) y[b * ystride + (int64_t)lane8 * n + r] = acc;
+#pragma unroll
+  for (int m = B; m < 8; m *= 2) acc = zadd(acc, shfl_xor_z(acc, m));
+  if (r < n && set == 0) y[b * ystride + (int64_t)col8 * n + r] = acc;
 }
 
-void launch_spmm8_il(int nb, int64_t n, const int64_t *rp, const int32_t *ci, const zd *vals, int64_t vstride,
-                     const zd *x, int64_t xstride, zd *xi, zd *y, int64_t ystride, hipStream_t s, KTime kt,
-                     bool xi_ready) {
-  if (!xi_ready) {
-    hipLaunchKernelGGL(k_interleave8, dim3((unsigned)((n + 255) / 256), nb), dim3(256), 0, s, n, x, xstride, xi,
-                       8 * n);
-    EMU_LAUNCH_CHECK();
-  }
+void launch_spmm_il(int nb, int64_t n, int bq, const int64_t *rp, const int32_t *ci, const zd *vals, int64_t vstride,
+                    const zd *x, int64_t xstride, zd *xi, zd *y, int64_t ystride, hipStream_t s, KTime kt,
+                    bool xi_ready) {
   const int per = (int)(((n + 31) / 32 + 7) / 8);
-  hipExtLaunchKernelGGL(k_spmm_il, dim3((unsigned)(8 * per), nb), dim3(256), 0, s, kt.a, kt.b, 0, n, rp, ci, vals,
-                        vstride, xi, 8 * n, y, ystride, per);
+  const dim3 gi((unsigned)((n + 255) / 256), nb), g((unsigned)(8 * per), nb);
+#define EMU_SPMM_IL(B)                                                                                               \
+  do {                                                                                                               \
+    if (!xi_ready) hipLaunchKernelGGL(k_interleave<B>, gi, dim3(256), 0, s, n, x, xstride, xi, B * n);               \
+    hipExtLaunchKernelGGL(k_spmm_il<B>, g, dim3(256), 0, s, kt.a, kt.b, 0, n, rp, ci, vals, vstride, xi, B * n, y,   \
+                          ystride, per);                                                                             \
+  } while (0)
+  switch (bq) {
+    case 2: EMU_SPMM_IL(2); break;
+    case 4: EMU_SPMM_IL(4); break;
+    case 8: EMU_SPMM_IL(8); break;
+    default: throw HipError("spmm_il: block size must be 2, 4 or 8");
+  }
+#undef EMU_SPMM_IL
   EMU_LAUNCH_CHECK();
 }
 
@@ -493,22 +509,19 @@ void launch_swap_i32(int64_t n, int32_t *a, int32_t *b, hipStream_t s) {
 }
 
 
-// The 16-column projection on the matrix cores: op(A)^T B with B of 16
-// columns, as four real v_mfma_f64_16x16x4f64 per 16 x 16 x 4 complex block
-// (real and imaginary parts).  A workgroup stages a 32-row x 64-column tile
-// of A and the 32 x 16 tile of B in LDS (as k_atb_tall); wave w multiplies
-// rows 8w .. 8w + 7 of the tile (two k-steps of 4) into four 16 x 16 output
-// tiles and writes its own partial product (four partials per K chunk, added
-// by k_atb_reduce).  Fragment layouts (FP64 16x16x4): A[i][k] in lane
-// i + 16 k, B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 (i % 4),
-// register i / 4.
-
-template <bool CONJ>
+// The projection of the delayed Gram-Schmidt on the matrix cores: A^H B with B
+// of N <= 16 columns (padded with zeros to 16), as four real
+// v_mfma_f64_16x16x4f64 per 16 x 16 x 4 complex block (real and imaginary
+// parts).  A workgroup stages a 32-row x 64-column tile of A and the 32 x 16
+// tile of B in LDS (as k_atb_tall); wave w multiplies rows 8w .. 8w + 7 of the
+// tile (two k-steps of 4) into four 16 x 16 output tiles, and the waves' sums
+// are added through LDS at the end (one partial per K chunk, added by
+// k_atb_reduce).  Fragment layouts (FP64 16x16x4): A[i][k] in lane i + 16 k,
+// B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 (i % 4), register i / 4.
 // three waves per SIMD (164 registers, no spills): more loads in flight
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void k_atb_mfma16(int64_t K, int M, int64_t kchunk, const zd *__restrict__ A,
-                                                    int64_t lda, int64_t sA, const zd *__restrict__ B, int64_t ldb,
-                                                    int64_t sB, zd *__restrict__ part) {
+void k_atb_mfma16(int64_t K, int M, int N, int64_t kchunk, const zd *__restrict__ A, int64_t lda, int64_t sA,
+                  const zd *__restrict__ B, int64_t ldb, int64_t sB, zd *__restrict__ part) {
   constexpr int TM = 64, TK = 32, NQ = 16;
   // The column tiles of one (K chunk, instance) all read the same rows of B.
   // Workgroups go to the 8 XCDs round-robin by linear id, each XCD with its
@@ -542,7 +555,7 @@ void k_atb_mfma16(int64_t K, int M, int64_t kchunk, const zd *__restrict__ A,
 #pragma unroll
     for (int i = 0; i < 8; ++i) ra[i] = Ab[kc + (int64_t)min(m0 + lc + 8 * i, M - 1) * lda];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) rb[i] = Bb[kc + (int64_t)(lc + 8 * i) * ldb];
+    for (int i = 0; i < 2; ++i) rb[i] = Bb[kc + (int64_t)min(lc + 8 * i, N - 1) * ldb];
   };
   v4d pr[4], pi[4];
 #pragma unroll
@@ -558,7 +571,7 @@ void k_atb_mfma16(int64_t K, int M, int64_t kchunk, const zd *__restrict__ A,
 #pragma unroll
     for (int i = 0; i < 8; ++i) As[lr][lc + 8 * i] = (okk && m0 + lc + 8 * i < M) ? ra[i] : zmk(0, 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) Bs[lr][lc + 8 * i] = okk ? rb[i] : zmk(0, 0);
+    for (int i = 0; i < 2; ++i) Bs[lr][lc + 8 * i] = (okk && lc + 8 * i < N) ? rb[i] : zmk(0, 0);
     __syncthreads();
     if (k0 + TK < ke) fetch(k0 + TK);
 #pragma unroll
@@ -568,68 +581,29 @@ void k_atb_mfma16(int64_t K, int M, int64_t kchunk, const zd *__restrict__ A,
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const zd va = As[kk][16 * t + fi];
-        // CONJ: Re += ar br + ai bi, Im += ar bi - ai br; else Re += ar br - ai bi, Im += ar bi + ai br
+        // conjugated: Re += ar br + ai bi, Im += ar bi - ai br
         pr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(va.x, xb.x, pr[t], 0, 0, 0);
-        pr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(CONJ ? va.y : -va.y, xb.y, pr[t], 0, 0, 0);
+        pr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(va.y, xb.y, pr[t], 0, 0, 0);
         pi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(va.x, xb.y, pi[t], 0, 0, 0);
-        pi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(CONJ ? -va.y : va.y, xb.x, pi[t], 0, 0, 0);
+        pi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-va.y, xb.x, pi[t], 0, 0, 0);
       }
     }
   }
-  const int64_t pc = ((int64_t)b * nchunk + chunk) * 4 + wv;  // this wave's partial
+  // the four waves' sums, one output tile at a time through As (wave, register,
+  // lane: 1,024 of its 2,080 entries)
+  zd *red = &As[0][0];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + 16 * t + fk + 4 * r;
-      if (m < M) part[(pc * NQ + fi) * M + m] = zmk(pr[t][r], pi[t][r]);
-    }
-}
-
-// Gram matrix W^H W of an 8-column block (K x 8, ld ldw), partial sums per K
-// chunk (layout of k_atb_tall's partials).  A 256-row tile of W is staged in
-// LDS; thread (o, g) owns output o = (p, q) and sums rows g, g + 4, ... of the
-// tile, so every lane does useful work (the general tall kernel would keep
-// 56 of its 64 columns idle).
-constexpr int GR_TK = 256;
-
-__global__ __launch_bounds__(256) void k_gram8(int64_t K, int64_t kchunk, const zd *__restrict__ W, int64_t ldw,
-                                               int64_t sW, zd *__restrict__ part) {
-  constexpr int NQ = 8;
-  __shared__ zd Ws[GR_TK][NQ + 1];
-  const int chunk = blockIdx.x, nchunk = gridDim.x, b = blockIdx.y, tid = threadIdx.x;
-  const int o = tid % (NQ * NQ), g = tid / (NQ * NQ), p = o % NQ, q = o / NQ;
-  const zd *Wb = W + b * sW;
-  const int64_t kb = chunk * kchunk, ke = min(K, kb + kchunk);
-  zd rw[NQ];
-  auto fetch = [&](int64_t k0) {
-    const int64_t k = k0 + tid;
-    const bool ok = k < ke;
-    const int64_t kc = ok ? k : ke - 1;
-#pragma unroll
-    for (int c = 0; c < NQ; ++c) {
-      const zd v = Wb[kc + (int64_t)c * ldw];
-      rw[c] = ok ? v : zmk(0, 0);
-    }
-  };
-  zd acc = zmk(0, 0);
-  if (kb < ke) fetch(kb);
-  for (int64_t k0 = kb; k0 < ke; k0 += GR_TK) {
+  for (int t = 0; t < 4; ++t) {
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < NQ; ++c) Ws[tid][c] = rw[c];
+    for (int i = 0; i < 4; ++i) red[(wv * 4 + i) * 64 + lane] = zmk(pr[t][i], pi[t][i]);
     __syncthreads();
-    if (k0 + GR_TK < ke) fetch(k0 + GR_TK);
-#pragma unroll 8
-    for (int kk = g; kk < GR_TK; kk += 4) acc = zfma(zconj(Ws[kk][p]), Ws[kk][q], acc);
-  }
-  __syncthreads();
-  zd *red = &Ws[0][0];
-  red[tid] = acc;
-  __syncthreads();
-  if (tid < NQ * NQ) {
-    const zd v = zadd(zadd(red[tid], red[tid + 64]), zadd(red[tid + 128], red[tid + 192]));
-    part[(((int64_t)b * nchunk + chunk) * NQ + q) * NQ + p] = v;
+    // thread (register wv, lane) adds the waves' values of that entry
+    zd sum = red[wv * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) sum = zadd(sum, red[(w * 4 + wv) * 64 + lane]);
+    const int m = m0 + 16 * t + fk + 4 * wv;
+    if (m < M && fi < N) part[(((int64_t)b * nchunk + chunk) * N + fi) * M + m] = sum;
   }
 }
 
@@ -656,7 +630,7 @@ void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64
                 int64_t ldb, int64_t sB, zd *C, int64_t ldc, int64_t sC, bool conjA, zd *scratch,
                 size_t scratch_elems, hipStream_t s, KTime kt) {
   if (M <= 0 || N <= 0 || nb <= 0) return;
-  const bool tall = N == 1 || N == 2 || N == 4 || N == 8 || N == 16;
+  const bool tall = N == 1;
   if (!tall) {  // wide products (mode overlaps, J contractions): 64 x 64 MFMA tiles, split over K
     const int tilesM = (M + 63) / 64, tiles = tilesM * ((N + 63) / 64);
     const int64_t per = (int64_t)nb * M * N;
@@ -683,48 +657,8 @@ void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64
     EMU_LAUNCH_CHECK();
     return;
   }
-  if (M == 8 && N == 8 && conjA && A == B && lda == ldb && sA == sB) {  // Gram matrix of a block
-    const int64_t per = (int64_t)nb * 64;
-    int64_t nchunk = std::max<int64_t>(1, std::min<int64_t>(1024 / std::max(nb, 1), (K + GR_TK - 1) / GR_TK));
-    nchunk = std::min<int64_t>(nchunk, std::max<int64_t>(1, (int64_t)(scratch_elems / per)));
-    int64_t kchunk = (K + nchunk - 1) / nchunk;
-    kchunk = ((kchunk + GR_TK - 1) / GR_TK) * GR_TK;
-    nchunk = (K + kchunk - 1) / kchunk;
-    hipExtLaunchKernelGGL(k_gram8, dim3((unsigned)nchunk, nb), dim3(256), 0, s, kt.a, kt.b, 0, K, kchunk, A, lda, sA,
-                          scratch);
-    EMU_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_atb_reduce, dim3(1, nb), dim3(256), 0, s, 8, 8, (int)nchunk, scratch, C, ldc, sC);
-    EMU_LAUNCH_CHECK();
-    return;
-  }
-  if (N == 16) {  // matrix cores (four partials per K chunk, one per wave)
-    const int tiles = (M + 63) / 64;
-    const int64_t per = (int64_t)nb * M * N * 4;
-    const int64_t maxchunk = std::max<int64_t>(1, (int64_t)(scratch_elems / std::max<int64_t>(per, 1)));
-    int64_t nchunk = std::min<int64_t>(std::min<int64_t>(std::max<int64_t>(1, 2048 / std::max(1, tiles * nb)),
-                                                         maxchunk), (K + 31) / 32);
-    nchunk = std::max<int64_t>(1, std::min<int64_t>(nchunk, 256));
-    int64_t kchunk = (K + nchunk - 1) / nchunk;
-    kchunk = ((kchunk + 31) / 32) * 32;
-    nchunk = (K + kchunk - 1) / kchunk;
-    if ((size_t)(nchunk * per) > scratch_elems) throw HipError("atb: scratch too small");
-    // the kernel renumbers the linear id of the whole grid in 32 bits
-    if ((int64_t)tiles * nchunk * nb > 0xffffffffLL) throw HipError("atb: grid too large");
-    dim3 g((unsigned)tiles, (unsigned)nchunk, nb), t(256);
-    if (conjA)
-      hipExtLaunchKernelGGL(k_atb_mfma16<true>, g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB, scratch);
-    else
-      hipExtLaunchKernelGGL(k_atb_mfma16<false>, g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB, scratch);
-    EMU_LAUNCH_CHECK();
-    const int64_t tot = (int64_t)M * N;
-    hipLaunchKernelGGL(k_atb_reduce, dim3((unsigned)((tot + 63) / 64), nb), dim3(256), 0, s, M, N, (int)(nchunk * 4),
-                       scratch, C, ldc, sC);
-    EMU_LAUNCH_CHECK();
-    return;
-  }
-  const int cpt = 1;
-  const int kstep = 32 / cpt;
-  const int tiles = (M + 64 * cpt - 1) / (64 * cpt);
+  const int kstep = 32;
+  const int tiles = (M + 63) / 64;
   int64_t per = (int64_t)nb * M * N;
   int64_t maxchunk = std::max<int64_t>(1, (int64_t)(scratch_elems / std::max<int64_t>(per, 1)));
   int64_t want = std::max<int64_t>(1, 2048 / std::max(1, tiles * nb));
@@ -734,14 +668,9 @@ void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64
   kchunk = ((kchunk + kstep - 1) / kstep) * kstep;
   nchunk = (K + kchunk - 1) / kchunk;
   if ((size_t)(nchunk * per) > scratch_elems) throw HipError("atb: scratch too small");
-  const int cj = conjA ? 1 : 0;
   dim3 g((unsigned)tiles, (unsigned)nchunk, nb), t(256);
-  switch (N) {
-    case 1: hipExtLaunchKernelGGL(k_atb_tall<1, 1>, g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB, cj, scratch); break;
-    case 2: hipExtLaunchKernelGGL(k_atb_tall<2, 1>, g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB, cj, scratch); break;
-    case 4: hipExtLaunchKernelGGL(k_atb_tall<4, 1>, g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB, cj, scratch); break;
-    default: hipExtLaunchKernelGGL(k_atb_tall<8, 1>, g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB, cj, scratch); break;
-  }
+  hipExtLaunchKernelGGL((k_atb_tall<1, 1>), g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB,
+                        conjA ? 1 : 0, scratch);
   EMU_LAUNCH_CHECK();
   const int64_t tot = (int64_t)M * N;
   hipLaunchKernelGGL(k_atb_reduce, dim3((unsigned)((tot + 63) / 64), nb), dim3(256), 0, s, M, N, (int)nchunk,
@@ -749,6 +678,33 @@ void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64
   EMU_LAUNCH_CHECK();
 }
 
+
+// The delayed Gram-Schmidt projection: C[b] (M x N) = A[b]^H B[b] for N <= 16
+// on the matrix cores.  K is cut into enough chunks for about 2,048
+// workgroups, but at least 128 rows each: every chunk writes M x N partial
+// sums, which at 32 rows per chunk (n = 6,072, 2 instances) were more bytes
+// than the basis itself.
+void launch_proj(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64_t sA, const zd *B, int64_t ldb,
+                 int64_t sB, zd *C, int64_t ldc, int64_t sC, zd *scratch, size_t scratch_elems, hipStream_t s, KTime kt) {
+  if (N > 16) throw HipError("proj: at most 16 columns");
+  const int tiles = (M + 63) / 64;
+  const int64_t per = (int64_t)nb * M * N;
+  int64_t nchunk = std::max<int64_t>(1, 2048 / std::max(1, tiles * nb));
+  nchunk = std::min<int64_t>({nchunk, (int64_t)(scratch_elems / std::max<int64_t>(per, 1)), (K + 127) / 128, 256});
+  nchunk = std::max<int64_t>(1, nchunk);
+  int64_t kchunk = (K + nchunk - 1) / nchunk;
+  kchunk = ((kchunk + 31) / 32) * 32;
+  nchunk = (K + kchunk - 1) / kchunk;
+  if ((size_t)(nchunk * per) > scratch_elems) throw HipError("proj: scratch too small");
+  // the kernel renumbers the linear id of the whole grid in 32 bits
+  if ((int64_t)tiles * nchunk * nb > 0xffffffffLL) throw HipError("proj: grid too large");
+  hipExtLaunchKernelGGL(k_atb_mfma16, dim3((unsigned)tiles, (unsigned)nchunk, nb), dim3(256), 0, s, kt.a, kt.b, 0, K, M,
+                        N, kchunk, A, lda, sA, B, ldb, sB, scratch);
+  EMU_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_atb_reduce, dim3((unsigned)(((int64_t)M * N + 63) / 64), nb), dim3(256), 0, s, M, N,
+                     (int)nchunk, scratch, C, ldc, sC);
+  EMU_LAUNCH_CHECK();
+}
 
 // ------------------------------------------------ C = alpha A B + beta C (NN)
 // Batched complex GEMM on the FP64 matrix cores, for the restart combination
@@ -1138,31 +1094,99 @@ void launch_sub_vh_blk(int nb, int64_t n, int k, int bq, const zd *V, int64_t ld
 // and a single read of the basis Vt = V[:, :j] gives both Vt^H Z (Z's
 // reorthogonalisation) and Vt^H W (W = OP Z's first projection), so each
 // block costs two passes over the basis instead of four.  The Arnoldi
-// relation OP V[:, :j] = V[:, :j+8] H[:j+8, :j] is kept exact by correcting
+// relation OP V[:, :j] = V[:, :j+B] H[:j+B, :j] is kept exact by correcting
 // row block j of H when Z is reorthogonalised and by removing OP Vt S (known
-// from H) from W.
+// from H) from W.  B = 2, 4 or 8 columns per block.
+//
+// One step's small dense work is spread over the row blocks of the basis
+// (k_dcgs_pre, k_dcgs_coef) and the Gram matrices of Cholesky-QR are formed
+// by the kernels that write the block (k_combine, k_trmm_right): at a few
+// thousand unknowns the step is a chain of launches of a few microseconds
+// each, and at 100,000 these kernels still take their time one after the
+// other.  Measured per step of 8 columns without the projection and the update
+// themselves (500-triangle cell, 2 instances / 8,000-triangle cell, 2
+// instances): 49 / 100 us, from 165 / 310 us with one workgroup per instance
+// for the coefficients, sequential 8 x 8 factorisations, a tiled GEMM for H S
+// and separate Gram and copy kernels.
+
+// Rows of the basis per workgroup in k_dcgs_pre and k_dcgs_coef.
+constexpr int DR = 32;
+
+// Gram matrix of B columns over the rows of a 256-thread workgroup, row r held
+// by thread r's w (gram_thread_rows) or already in ws.  The
+// rows are staged 128 at a time (18 KB of LDS at B = 8): thread (p + B q, g) sums conj(w_p) w_q over rows g,
+// g + G, ..., and the G partial sums are added pairwise.  Threads < B^2 return
+// output p + B q.
+constexpr int GR = 128;
+template <int B>
+struct GramLds {
+  zd ws[GR][B + 1];
+  zd red[256];
+};
+template <int B>
+__device__ __forceinline__ zd gram_acc(const GramLds<B> &g, int rows, zd acc) {
+  constexpr int G = 256 / (B * B);
+  const int tid = threadIdx.x, o = tid % (B * B), p = o % B, q = o / B;
+#pragma unroll 8
+  for (int r = tid / (B * B); r < rows; r += G) acc = zcfma(g.ws[r][p], g.ws[r][q], acc);
+  return acc;
+}
+template <int B>
+__device__ __forceinline__ zd gram_sum(GramLds<B> &g, zd acc) {
+  constexpr int G = 256 / (B * B);
+  const int tid = threadIdx.x, o = tid % (B * B);
+  g.red[tid] = acc;
+#pragma unroll
+  for (int h = G / 2; h > 0; h /= 2) {
+    __syncthreads();
+    if (tid < h * B * B) g.red[tid] = zadd(g.red[tid], g.red[tid + h * B * B]);
+  }
+  return g.red[o];  // threads < B^2 read what they wrote
+}
+template <int B>
+__device__ __forceinline__ zd gram_thread_rows(GramLds<B> &g, const zd *w) {
+  zd acc = zmk(0, 0);
+#pragma unroll
+  for (int h = 0; h < 256; h += GR) {
+    if (h > 0) __syncthreads();
+    if ((int)threadIdx.x >= h && (int)threadIdx.x < h + GR)
+#pragma unroll
+      for (int q = 0; q < B; ++q) g.ws[threadIdx.x - h][q] = w[q];
+    __syncthreads();
+    acc = gram_acc<B>(g, GR, acc);
+  }
+  return gram_sum<B>(g, acc);
+}
 
 // W[b] (n x NQ, in place) = W[b] L[b] - V[b][:, :k] E[b] (L: NQ x NQ, column-
 // major; E: k x NQ, row-major so that the NQ coefficients of basis column c
-// are contiguous).  Thread per row.  The coefficients of a column are the
-// same for every lane, so they are read with scalar loads straight into
-// SGPRs and used as FMA operands: no LDS traffic in the main loop.
-template <int NQ>
+// are contiguous).  The coefficients of a column are the same for every lane,
+// so they are read with scalar loads straight into SGPRs and used as FMA
+// operands: no LDS traffic in the main loop.  GRAM: also the Gram matrix of
+// the last NQ / 2 columns over the workgroup's rows, gpart[b][block].
+// QS = 1: a thread per row (bandwidth-bound on V).  QS = 4: 64 rows per
+// workgroup and NQ / 4 columns per wave, for problems whose rows alone leave
+// most SIMDs idle: a row's NQ FMAs per basis column are a serial stream of
+// 256 clocks at NQ = 16.
+template <int NQ, int QS, bool GRAM>
 __global__ __launch_bounds__(256) void k_combine(int64_t n, int k, const zd *__restrict__ V, int64_t ldv,
                                                  int64_t sV, const zd *__restrict__ E, int64_t sE,
                                                  const zd *__restrict__ L, zd *__restrict__ W, int64_t ldw,
-                                                 int64_t sW) {
+                                                 int64_t sW, zd *__restrict__ gpart) {
+  constexpr int R = 256 / QS, C = NQ / QS, B = NQ / 2;
   __shared__ zd ls[NQ][NQ];
   const int b = blockIdx.y;
-  const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t rr = r < n ? r : n - 1;  // clamped row: loads stay in bounds, the store is skipped
+  const int lrow = threadIdx.x % R;
+  const int q0 = QS == 1 ? 0 : C * __builtin_amdgcn_readfirstlane(threadIdx.x / R);
+  const int r = blockIdx.x * R + lrow, nr = (int)n;  // n < 2^31 (checked by the launcher)
+  const int rr = min(r, nr - 1);                     // clamped row: loads stay in bounds, the store is skipped
   const zd *Vb = V + b * sV + rr;
-  const zd *Eb = E + b * sE;
+  const zd *Eb = E + b * sE + q0;
   for (int idx = threadIdx.x; idx < NQ * NQ; idx += blockDim.x) ls[idx % NQ][idx / NQ] = L[(int64_t)b * NQ * NQ + idx];
   __syncthreads();
-  zd acc[NQ];
+  zd acc[C];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) acc[q] = zmk(0, 0);
+  for (int q = 0; q < C; ++q) acc[q] = zmk(0, 0);
   // acc = W L, W read in halves of NQ / 2 columns, each half's loads all in
   // flight before the first use (the scheduler would otherwise wait for each
   // in turn); halves keep the live registers within four waves per SIMD
@@ -1173,342 +1197,544 @@ __global__ __launch_bounds__(256) void k_combine(int64_t n, int k, const zd *__r
     for (int p = 0; p < NQ / 2; ++p) x[p] = W[b * sW + (h + p) * ldw + rr];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
+    for (int q = 0; q < C; ++q)
 #pragma unroll
-      for (int p = 0; p < NQ / 2; ++p) acc[q] = zfma(x[p], ls[h + p][q], acc[q]);
+      for (int p = 0; p < NQ / 2; ++p) acc[q] = zfma(x[p], ls[h + p][q0 + q], acc[q]);
   }
-#pragma unroll 2
+  if (QS > 1) __syncthreads();  // W is read by every wave before any writes it
+#pragma unroll QS == 1 ? 2 : 8
   for (int c = 0; c < k; ++c) {
     const zd v = Vb[(int64_t)c * ldv];
     const zd *ec = Eb + (int64_t)c * NQ;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) acc[q] = zfms(v, ec[q], acc[q]);
+    for (int q = 0; q < C; ++q) acc[q] = zfms(v, ec[q], acc[q]);
   }
-  if (r < n)
+  if (r < nr)
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) W[b * sW + q * ldw + r] = acc[q];
-}
-
-void launch_combine(int nb, int64_t n, int k, int nq, const zd *V, int64_t ldv, int64_t sV, const zd *E,
-                    int64_t sE, const zd *L, zd *W, int64_t ldw, int64_t sW, hipStream_t s, KTime kt) {
-  dim3 g((unsigned)((n + 255) / 256), nb), t(256);
-  switch (nq) {
-    case 8: hipExtLaunchKernelGGL(k_combine<8>, g, t, 0, s, kt.a, kt.b, 0, n, k, V, ldv, sV, E, sE, L, W, ldw, sW); break;
-    case 16: hipExtLaunchKernelGGL(k_combine<16>, g, t, 0, s, kt.a, kt.b, 0, n, k, V, ldv, sV, E, sE, L, W, ldw, sW); break;
-    default: throw HipError("combine: 8 or 16 columns");
+    for (int q = 0; q < C; ++q) W[b * sW + (q0 + q) * ldw + r] = acc[q];
+  if constexpr (GRAM) {
+    static_assert(R <= GR, "the workgroup's rows fit the staging");
+    __shared__ GramLds<B> gl;
+    if (r >= nr)
+#pragma unroll
+      for (int q = 0; q < C; ++q) acc[q] = zmk(0, 0);
+#pragma unroll
+    for (int q = 0; q < C; ++q)
+      if (q0 + q >= B) gl.ws[lrow][q0 + q - B] = acc[q];
+    __syncthreads();
+    const zd g = gram_sum<B>(gl, gram_acc<B>(gl, R, zmk(0, 0)));
+    if (threadIdx.x < B * B) gpart[((int64_t)b * gridDim.x + blockIdx.x) * B * B + threadIdx.x] = g;
   }
-  EMU_LAUNCH_CHECK();
 }
 
-// Coefficients of one delayed step, one workgroup per instance (block size 8).
-//   P = [Vt Z W]^H [Z W] ((j + 16) x 16, ld ldp): S = P[:j, :8], T = P[:j, 8:],
-//   G = P[j:j+16, :] = [Z W]^H [Z W];  A0 = H[:j, :j] S (j x 8, ld lda), old H
-//   row block j of H (rows j..j+7) is nonzero in columns [c0, j)
+// Split columns where the rows alone fill at most about one wave per SIMD
+// (1,024 SIMDs); NQ = 16, split against not: 190 waves (n = 6,072, 2 instances)
+// 14 / 36 us, 1,116 waves (n = 17,832, 4) 46 / 70 us, 3,006 waves (n = 96,168,
+// 2) 267 / 202 us.
+// Only the split form adds the Gram matrix: with it the other one needs a
+// 129th register, hence three instead of four waves per SIMD (805 -> 1,340 us
+// at 96,168 unknowns and 8 instances), while k_gram takes 24 us there.
+int64_t launch_combine(int nb, int64_t n, int k, int nq, const zd *V, int64_t ldv, int64_t sV, const zd *E,
+                       int64_t sE, const zd *L, zd *W, int64_t ldw, int64_t sW, zd *gpart, hipStream_t s, KTime kt) {
+  if (n > INT32_MAX - 256) throw HipError("combine: too many rows");
+  const bool split = nq >= 4 && (n + 63) / 64 * nb <= 1280;
+  const unsigned blocks = (unsigned)(split ? (n + 63) / 64 : (n + 255) / 256);
+  dim3 g(blocks, nb), t(256);
+#define EMU_COMBINE(NQ, QS, GR) \
+  hipExtLaunchKernelGGL((k_combine<NQ, QS, GR>), g, t, 0, s, kt.a, kt.b, 0, n, k, V, ldv, sV, E, sE, L, W, ldw, sW, gpart)
+#define EMU_COMBINE_NQ(NQ)                    \
+  if (!split) EMU_COMBINE(NQ, 1, false);      \
+  else if (gpart) EMU_COMBINE(NQ, 4, true);   \
+  else EMU_COMBINE(NQ, 4, false);
+  switch (nq) {
+    case 2: EMU_COMBINE(2, 1, false); break;
+    case 4: EMU_COMBINE_NQ(4) break;
+    case 8: EMU_COMBINE_NQ(8) break;
+    case 16: EMU_COMBINE_NQ(16) break;
+    default: throw HipError("combine: 2, 4, 8 or 16 columns");
+  }
+#undef EMU_COMBINE_NQ
+#undef EMU_COMBINE
+  EMU_LAUNCH_CHECK();
+  return split && gpart ? blocks : 0;
+}
+
+// Cholesky factor R (upper, real diagonal) of the B x B Gram matrix C and its
+// inverse, by one wavefront: lane p + B q holds entry (p, q), each of the B
+// steps is a few cross-lane moves.  A non-positive pivot (rank-deficient block)
+// is replaced by a tiny value and counted.
+template <int B>
+__device__ __forceinline__ int chol_inv(zd c, double gmax, int lane, zd &R, zd &Ri) {
+  const int p = lane % B, q = (lane / B) % B;
+  int nbad = 0;
+  R = zmk(0, 0);
+  double dinv[B];
+#pragma unroll
+  for (int k = 0; k < B; ++k) {
+    double d = __shfl(c.x, k + B * k, 64);
+    if (!(d > 1e-28 * gmax)) {
+      d = 1e-28 * gmax + 1e-300;
+      ++nbad;
+    }
+    const double rk = sqrt(d);
+    dinv[k] = 1.0 / rk;
+    const zd cp = shfl_z(c, k + B * p), cq = shfl_z(c, k + B * q);  // row k of C at columns p and q
+    const zd rp = zscale(cp, dinv[k]), rq = zscale(cq, dinv[k]);
+    if (p == k && q == k) R = zmk(rk, 0.0);
+    else if (p == k && q > k) R = rq;
+    else if (p > k && q > k) c = zsub(c, zmul(zconj(rp), rq));
+  }
+  // X = R^-1: rows from the last; acc = (delta - sum over finished rows)
+  Ri = zmk(p == q ? 1.0 : 0.0, 0.0);
+#pragma unroll
+  for (int k = B - 1; k >= 0; --k) {
+    if (p == k) Ri = zscale(Ri, dinv[k]);
+    const zd xk = shfl_z(Ri, k + B * q), rik = shfl_z(R, p + B * k);
+    if (p < k) Ri = zfms(rik, xk, Ri);
+  }
+  if (p > q) Ri = zmk(0, 0);
+  return nbad;
+}
+
+// First half of a step's coefficients: per 32 rows i of the basis,
+//   A0[i, :] = H[i, :j] S,
+// and over these rows the partial sums of S^H S, S^H T and u = H[j:j+B, c0:j] S
+// (part[b][block][3][B][B], row index first).  P = [Vt Z W]^H [Z W]
+// ((j + 2B) x 2B, ld ldp): S = P[:j, :B], T = P[:j, B:].  FIN (P = [Vt Z]^H Z):
+// S^H S only.
+template <int B, bool FIN>
+__global__ __launch_bounds__(256) void k_dcgs_pre(int j, int c0, const zd *__restrict__ P, int64_t ldp, int64_t sP,
+                                                  const zd *__restrict__ H, int64_t ldh, int64_t sH,
+                                                  zd *__restrict__ A0, int64_t lda, int64_t sA,
+                                                  zd *__restrict__ part) {
+  constexpr int KG = 256 / DR, KB = 64;  // k groups, k per round
+  const int b = blockIdx.y, tid = threadIdx.x, i0 = blockIdx.x * DR;
+  const zd *Pb = P + b * sP, *Hb = H + b * sH;
+  __shared__ zd Ps[DR][2 * B + 1], Hr[B][DR + 1];
+  for (int idx = tid; idx < DR * 2 * B; idx += 256) {
+    const int r = idx % DR, c = idx / DR;
+    const zd v = Pb[min(i0 + r, j - 1) + (int64_t)(FIN ? c % B : c) * ldp];
+    Ps[r][c] = i0 + r < j ? v : zmk(0, 0);
+  }
+  if (!FIN)
+    for (int idx = tid; idx < DR * B; idx += 256) {
+      const int p = idx % B, r = idx / B, c = i0 + r;
+      const zd v = Hb[j + p + (int64_t)min(c, j - 1) * ldh];
+      Hr[p][r] = (c >= c0 && c < j) ? v : zmk(0, 0);
+    }
+  __syncthreads();
+  for (int o = tid; o < (FIN ? 1 : 3) * B * B; o += 256) {
+    const int which = o / (B * B), p = o % B, q = o / B % B;
+    zd acc = zmk(0, 0);
+#pragma unroll 8
+    for (int r = 0; r < DR; ++r) {
+      if (which == 2) acc = zfma(Hr[p][r], Ps[r][q], acc);
+      else acc = zcfma(Ps[r][p], Ps[r][which * B + q], acc);
+    }
+    part[(((int64_t)b * gridDim.x + blockIdx.x) * 3 + which) * B * B + p + B * q] = acc;
+  }
+  if (FIN) return;
+  // A0: thread (row r, group g) sums k = g, g + KG, ... of every round
+  __shared__ zd Ss[KB][B + 1];
+  __shared__ zd red[KG][DR][B + 1];
+  const int r = tid % DR, g = tid / DR;
+  zd acc[B];
+#pragma unroll
+  for (int q = 0; q < B; ++q) acc[q] = zmk(0, 0);
+  for (int k0 = 0; k0 < j; k0 += KB) {
+    zd h[KB / KG];
+#pragma unroll
+    for (int u = 0; u < KB / KG; ++u) h[u] = Hb[min(i0 + r, j - 1) + (int64_t)min(k0 + g + KG * u, j - 1) * ldh];
+    __syncthreads();
+    for (int idx = tid; idx < KB * B; idx += 256) {
+      const int k = idx % KB, q = idx / KB;
+      const zd v = Pb[min(k0 + k, j - 1) + (int64_t)q * ldp];
+      Ss[k][q] = k0 + k < j ? v : zmk(0, 0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < KB / KG; ++u)
+#pragma unroll
+      for (int q = 0; q < B; ++q) acc[q] = zfma(h[u], Ss[g + KG * u][q], acc[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < B; ++q) red[g][r][q] = acc[q];
+  __syncthreads();
+  for (int idx = tid; idx < DR * B; idx += 256) {
+    const int rr = idx % DR, q = idx / DR;
+    zd v = red[0][rr][q];
+#pragma unroll
+    for (int k = 1; k < KG; ++k) v = zadd(v, red[k][rr][q]);
+    if (i0 + rr < j) A0[b * sA + i0 + rr + (int64_t)q * lda] = v;
+  }
+}
+
+// Second half, one workgroup per 32 rows of the basis (at least one):
+//   G = P[j:j+2B, :] = [Z W]^H [Z W];  row block j of H (rows j .. j+B-1) is
+//   nonzero in columns [c0, j).
 // Z's reorthogonalisation: C = Z^H Z - S^H S = R^H R, Q = (Z - Vt S) R^-1,
-// H[:j, c0:j] += S H[j:j+8, c0:j], H[j:j+8, c0:j] = R H[j:j+8, c0:j].
+// H[:j, c0:j] += S H[j:j+B, c0:j], H[j:j+B, c0:j] <- R H[j:j+B, c0:j].
 // W's first projection against [Vt, Q] with OP Vt S = [Vt, Q] H S removed:
-//   u = H_old[j:j+8, :j] S, a = A0 + S u, b = R u,
+//   u = H_old[j:j+B, :j] S, a = A0 + S u, b = R u,
 //   cV = (T - a) R^-1, cQ = R^-H (Z^H W - S^H T) R^-1 - b R^-1  (column j of H),
 //   D = b R^-1 + cQ, E = [S R^-1, a R^-1 + cV - S R^-1 D],
 //   L = [[R^-1, -R^-1 D], [0, R^-1]], so that [Q, Zraw] = [Z W] L - Vt E.
 // FIN (no W; the last provisional block of an expansion; P = [Vt Z]^H Z):
-// only Z's reorthogonalisation, E = S R^-1 (j x 8), L = R^-1.
-template <bool FIN>
+// only Z's reorthogonalisation, E = S R^-1 (j x B), L = R^-1.
+// Every workgroup forms the B x B quantities for itself (a few microseconds,
+// less than another launch) and applies them to its rows; R H[j:j+B, c0:j] goes
+// to Hrow (B x j) because the other workgroups read the old rows: k_cholqr
+// (or, FIN, k_hrow) stores it.
+template <int B, bool FIN>
 __global__ __launch_bounds__(256) void k_dcgs_coef(int j, int c0, const zd *__restrict__ P, int64_t ldp, int64_t sP,
-                                                   const zd *__restrict__ A0, int64_t lda,
-                                                   int64_t sA, zd *__restrict__ H, int64_t ldh, int64_t sH,
-                                                   zd *__restrict__ E, int64_t sE, zd *__restrict__ L,
+                                                   const zd *__restrict__ A0, int64_t lda, int64_t sA,
+                                                   const zd *__restrict__ part, int nblk, zd *__restrict__ H,
+                                                   int64_t ldh, int64_t sH, zd *__restrict__ E, int64_t sE,
+                                                   zd *__restrict__ L, zd *__restrict__ Hrow, int64_t sR,
                                                    int32_t *__restrict__ bad) {
-  constexpr int B = 8;
-  constexpr int NG = FIN ? B : 2 * B;
-  const int b = blockIdx.x, tid = threadIdx.x;
+  constexpr int NG = FIN ? B : 2 * B, BB = B * B;
+  const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const zd *Pb = P + b * sP;
   zd *Hb = H + b * sH;
   zd *Eb = E + b * sE;
-  __shared__ zd SS[B][B], ST[B][B], U[B][B], R[B][B], Ri[B][B], Bm[B][B], CQ[B][B], Dm[B][B], T1[B][B];
-  __shared__ zd Gs[NG][NG];
-  for (int idx = tid; idx < NG * NG; idx += blockDim.x) Gs[idx % NG][idx / NG] = Pb[(j + idx % NG) + (idx / NG) * ldp];
-  // 1. S^H S, S^H T over the j basis rows: 32-row chunks of P[:, :16] are
-  // staged in LDS by all threads (row tid % 32, columns tid / 32 and
-  // tid / 32 + 8), so a chunk costs one round of loads; one thread per
-  // output then sums the chunk's rows in order (the same order, hence the
-  // same rounding, as a single loop over i).  u = Hrow S after the loop.
-  __shared__ zd Pc[32][2 * B + 1];
-  {
-    const int o = tid % (B * B), kind = tid / (B * B), p = o % B, q = o / B;
-    const int lr = tid & 31, lc = tid >> 5;
+  __shared__ zd Gs[NG][NG], S3[3][BB], R[B][B], Ri[B][B], Bm[B][B], Dm[B][B], T1[B][B], T2[B][B];
+  for (int idx = tid; idx < NG * NG; idx += 256) Gs[idx % NG][idx / NG] = Pb[(j + idx % NG) + (int64_t)(idx / NG) * ldp];
+  for (int o = tid; o < (FIN ? 1 : 3) * BB; o += 256) {
+    const zd *pp = part + (int64_t)b * nblk * 3 * BB + o;
     zd acc = zmk(0, 0);
-    for (int i0 = 0; i0 < j; i0 += 32) {
-      const int i = i0 + lr;
-      const bool ok = i < j;
-      const zd v0 = ok ? Pb[i + lc * ldp] : zmk(0, 0);
-      const zd v1 = (ok && !FIN) ? Pb[i + (lc + B) * ldp] : zmk(0, 0);
-      __syncthreads();  // the previous chunk has been consumed
-      Pc[lr][lc] = v0;
-      Pc[lr][lc + B] = v1;
-      __syncthreads();
-      if (kind < 2) {
-        const int nr = min(32, j - i0), cq = kind == 0 ? q : B + q;
-        for (int rr = 0; rr < nr; ++rr) acc = zfma(zconj(Pc[rr][p]), Pc[rr][cq], acc);
-      }
+    for (int k = 0; k < nblk; k += 4) {
+      zd v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = pp[(int64_t)min(k + u, nblk - 1) * 3 * BB];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (k + u < nblk) acc = zadd(acc, v[u]);
     }
-    if (kind == 0) SS[p][q] = acc;
-    if (kind == 1) ST[p][q] = FIN ? zmk(0, 0) : acc;
-  }
-  if (tid >= 2 * B * B && tid < 3 * B * B) {
-    const int o = tid % (B * B), p = o % B, q = o / B;
-    zd acc = zmk(0, 0);
-    {
-      if (!FIN) {
-#pragma unroll 8
-        for (int c = c0; c < j; ++c) acc = zfma(Hb[(j + p) + (int64_t)c * ldh], Pb[c + q * ldp], acc);
-      }
-      U[p][q] = acc;
-    }
+    S3[o / BB][o % BB] = acc;
   }
   __syncthreads();
-  // 2. Cholesky of C = Z^H Z - S^H S and the inverse of R (one thread)
-  if (tid == 0) {
+  const int p = lane % B, q = lane / B % B;
+  if (tid < 64) {
     double gmax = 0;
+#pragma unroll
     for (int i = 0; i < B; ++i) gmax = fmax(gmax, Gs[i][i].x);
-    for (int c = 0; c < B; ++c) {
-      for (int i = 0; i < B; ++i) { R[i][c] = zmk(0, 0); Ri[i][c] = zmk(0, 0); }
+    zd r, ri;
+    const int nbad = chol_inv<B>(zsub(Gs[p][q], S3[0][p + B * q]), gmax, lane, r, ri);
+    if (lane < BB) {
+      R[p][q] = r;
+      Ri[p][q] = ri;
     }
-    for (int c = 0; c < B; ++c) {
-      for (int i = 0; i < c; ++i) {
-        zd acc = zsub(Gs[i][c], SS[i][c]);
-        for (int k = 0; k < i; ++k) acc = zsub(acc, zmul(zconj(R[k][i]), R[k][c]));
-        R[i][c] = zdiv(acc, R[i][i]);
-      }
-      double d = Gs[c][c].x - SS[c][c].x;
-      for (int k = 0; k < c; ++k) d -= R[k][c].x * R[k][c].x + R[k][c].y * R[k][c].y;
-      if (!(d > 1e-28 * gmax)) {
-        d = 1e-28 * gmax + 1e-300;
-        bad[b] += 1;
-      }
-      R[c][c] = zmk(sqrt(d), 0);
-    }
-    for (int c = 0; c < B; ++c) {
-      Ri[c][c] = zdiv(zmk(1, 0), R[c][c]);
-      for (int i = c - 1; i >= 0; --i) {
-        zd acc = zmk(0, 0);
-        for (int k = i + 1; k <= c; ++k) acc = zadd(acc, zmul(R[i][k], Ri[k][c]));
-        Ri[i][c] = zsub(zmk(0, 0), zdiv(acc, R[i][i]));
-      }
-    }
+    if (tid == 0 && blockIdx.x == 0 && nbad) bad[b] += nbad;
   }
   __syncthreads();
-  // 3. b = R u; T1 = Z^H W - S^H T; CQ = Ri^H T1 Ri - b Ri; D = Ri^H T1 Ri (64 threads, one entry each)
-  const int p8 = tid % B, q8 = (tid / B) % B;
   if (!FIN) {
-    if (tid < B * B) {
+    if (tid < BB) {
       zd acc = zmk(0, 0);
-      for (int k = p8; k < B; ++k) acc = zfma(R[p8][k], U[k][q8], acc);
-      Bm[p8][q8] = acc;
-      T1[p8][q8] = zsub(Gs[p8][B + q8], ST[p8][q8]);
+      for (int k = p; k < B; ++k) acc = zfma(R[p][k], S3[2][k + B * q], acc);
+      Bm[p][q] = acc;  // b = R u
+      T1[p][q] = zsub(Gs[p][B + q], S3[1][p + B * q]);
     }
     __syncthreads();
-    if (tid < B * B) {  // SS reused: T1 Ri
+    if (tid < BB) {
       zd acc = zmk(0, 0);
-      for (int k = 0; k <= q8; ++k) acc = zfma(T1[p8][k], Ri[k][q8], acc);
-      SS[p8][q8] = acc;
+      for (int k = 0; k <= q; ++k) acc = zfma(T1[p][k], Ri[k][q], acc);
+      T2[p][q] = acc;
     }
     __syncthreads();
-    if (tid < B * B) {
+    if (tid < BB) {
       zd acc = zmk(0, 0), bri = zmk(0, 0);
-      for (int k = 0; k <= p8; ++k) acc = zfma(zconj(Ri[k][p8]), SS[k][q8], acc);
-      for (int k = 0; k <= q8; ++k) bri = zfma(Bm[p8][k], Ri[k][q8], bri);
-      CQ[p8][q8] = zsub(acc, bri);
-      Dm[p8][q8] = acc;  // D = b R^-1 + cQ = R^-H T1 R^-1
+      for (int k = 0; k <= p; ++k) acc = zcfma(Ri[k][p], T2[k][q], acc);
+      for (int k = 0; k <= q; ++k) bri = zfma(Bm[p][k], Ri[k][q], bri);
+      Dm[p][q] = acc;                                                 // D = R^-H T1 R^-1
+      if (blockIdx.x == 0) Hb[(j + p) + (int64_t)(j + q) * ldh] = zsub(acc, bri);  // cQ
     }
     __syncthreads();
   }
-  // 4. per basis row i < j: a, cV (column j of H), E.  32 rows at a time, one
-  // thread per (row, column); the row vectors a and S R^-1 go through LDS.
-  __shared__ zd sa[32][B], se[32][B];
-  {
-    const int rr = tid / B, q = tid % B;
-    for (int i0 = 0; i0 < j; i0 += 32) {
-      const int i = i0 + rr;
-      const bool ok = i < j;
-      zd e1 = zmk(0, 0), av = zmk(0, 0);
-      if (ok) {
-        for (int k = 0; k <= q; ++k) e1 = zfma(Pb[i + k * ldp], Ri[k][q], e1);
-        Eb[(int64_t)i * NG + q] = e1;
-        if (!FIN) {
-          av = A0[b * sA + i + (int64_t)q * lda];
-          for (int k = 0; k < B; ++k) av = zfma(Pb[i + k * ldp], U[k][q], av);
-        }
-      }
-      se[rr][q] = e1;
-      sa[rr][q] = av;
-      __syncthreads();
-      if (!FIN && ok) {
-        zd cv = zmk(0, 0), e2 = zmk(0, 0);
-        for (int k = 0; k <= q; ++k) {
-          cv = zfma(zsub(Pb[i + (B + k) * ldp], sa[rr][k]), Ri[k][q], cv);
-          e2 = zfma(sa[rr][k], Ri[k][q], e2);
-        }
-        for (int k = 0; k < B; ++k) e2 = zfms(se[rr][k], Dm[k][q], e2);
-        Hb[i + (int64_t)(j + q) * ldh] = cv;
-        Eb[(int64_t)i * NG + B + q] = zadd(e2, cv);
-      }
-      __syncthreads();
+  // this workgroup's rows: E, column block j of H, and the row correction
+  __shared__ zd Ps[DR][2 * B + 1], sa[DR][B], se[DR][B];
+  const int i0 = blockIdx.x * DR;
+  if (i0 < j) {
+    for (int idx = tid; idx < DR * NG; idx += 256) {
+      const int r = idx % DR, c = idx / DR;
+      Ps[r][c] = Pb[min(i0 + r, j - 1) + (int64_t)c * ldp];
     }
+    __syncthreads();
+    for (int idx = tid; idx < DR * B; idx += 256) {
+      const int rr = idx / B, c = idx % B, i = i0 + rr;
+      zd e1 = zmk(0, 0), av = zmk(0, 0);
+      for (int k = 0; k <= c; ++k) e1 = zfma(Ps[rr][k], Ri[k][c], e1);
+      if (i < j) Eb[(int64_t)i * NG + c] = e1;
+      if (!FIN) {
+        av = A0[b * sA + min(i, j - 1) + (int64_t)c * lda];
+#pragma unroll
+        for (int k = 0; k < B; ++k) av = zfma(Ps[rr][k], S3[2][k + B * c], av);
+      }
+      se[rr][c] = e1;
+      sa[rr][c] = av;
+    }
+    __syncthreads();
+    if (!FIN)
+      for (int idx = tid; idx < DR * B; idx += 256) {
+        const int rr = idx / B, c = idx % B, i = i0 + rr;
+        zd cv = zmk(0, 0), e2 = zmk(0, 0);
+        for (int k = 0; k <= c; ++k) {
+          cv = zfma(zsub(Ps[rr][B + k], sa[rr][k]), Ri[k][c], cv);
+          e2 = zfma(sa[rr][k], Ri[k][c], e2);
+        }
+#pragma unroll
+        for (int k = 0; k < B; ++k) e2 = zfms(se[rr][k], Dm[k][c], e2);
+        if (i < j) {
+          Hb[i + (int64_t)(j + c) * ldh] = cv;
+          Eb[(int64_t)i * NG + B + c] = zadd(e2, cv);
+        }
+      }
+    const int rr = tid % DR;
+    if (i0 + rr < j)
+      for (int c = c0 + tid / DR; c < j; c += 256 / DR) {
+        zd hr[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) hr[k] = Hb[(j + k) + (int64_t)c * ldh];
+        zd acc = Hb[i0 + rr + (int64_t)c * ldh];
+#pragma unroll
+        for (int k = 0; k < B; ++k) acc = zfma(Ps[rr][k], hr[k], acc);
+        Hb[i0 + rr + (int64_t)c * ldh] = acc;
+      }
   }
-  const int w = j - c0;
-  for (int64_t idx = tid; idx < (int64_t)j * w; idx += blockDim.x) {
-    const int i = (int)(idx % j), c = c0 + (int)(idx / j);
-    zd acc = Hb[i + (int64_t)c * ldh];
-    for (int k = 0; k < B; ++k) acc = zfma(Pb[i + k * ldp], Hb[(j + k) + (int64_t)c * ldh], acc);
-    Hb[i + (int64_t)c * ldh] = acc;
-  }
-  __syncthreads();
-  // 5. Hrow <- R Hrow, column j's diagonal block, L
-  for (int c = c0 + tid; c < j; c += blockDim.x) {
+  if (blockIdx.x != 0) return;
+  for (int c = c0 + tid; c < j; c += 256) {
     zd h[B];
 #pragma unroll
     for (int k = 0; k < B; ++k) h[k] = Hb[(j + k) + (int64_t)c * ldh];
 #pragma unroll
-    for (int p = 0; p < B; ++p) {
+    for (int i = 0; i < B; ++i) {
       zd acc = zmk(0, 0);
 #pragma unroll
-      for (int k = p; k < B; ++k) acc = zfma(R[p][k], h[k], acc);
-      Hb[(j + p) + (int64_t)c * ldh] = acc;
+      for (int k = i; k < B; ++k) acc = zfma(R[i][k], h[k], acc);
+      Hrow[b * sR + i + (int64_t)c * B] = acc;
     }
   }
   zd *Lb = L + (int64_t)b * NG * NG;
-  if (FIN) {
-    if (tid < B * B) Lb[p8 + q8 * B] = Ri[p8][q8];
-  } else {
-    if (tid < B * B) {
-      Hb[(j + p8) + (int64_t)(j + q8) * ldh] = CQ[p8][q8];
+  if (tid < BB) {
+    Lb[p + q * NG] = Ri[p][q];
+    if (!FIN) {
       zd rd = zmk(0, 0);
-      for (int k = p8; k < B; ++k) rd = zfma(Ri[p8][k], Dm[k][q8], rd);
-      Lb[p8 + q8 * NG] = Ri[p8][q8];
-      Lb[p8 + (B + q8) * NG] = zsub(zmk(0, 0), rd);
-      Lb[(B + p8) + q8 * NG] = zmk(0, 0);
-      Lb[(B + p8) + (B + q8) * NG] = Ri[p8][q8];
+      for (int k = p; k < B; ++k) rd = zfma(Ri[p][k], Dm[k][q], rd);
+      Lb[p + (B + q) * NG] = zsub(zmk(0, 0), rd);
+      Lb[(B + p) + q * NG] = zmk(0, 0);
+      Lb[(B + p) + (B + q) * NG] = Ri[p][q];
     }
   }
 }
 
-void launch_dcgs_coef(int nb, bool fin, int j, int c0, const zd *P, int64_t ldp, int64_t sP, const zd *A0,
-                      int64_t lda, int64_t sA, zd *H, int64_t ldh, int64_t sH, zd *E, int64_t sE, zd *L, int32_t *bad,
-                      hipStream_t s) {
-  if (fin)
-    hipLaunchKernelGGL(k_dcgs_coef<true>, dim3(nb), dim3(256), 0, s, j, c0, P, ldp, sP, A0, lda, sA, H, ldh, sH, E, sE,
-                       L, bad);
-  else
-    hipLaunchKernelGGL(k_dcgs_coef<false>, dim3(nb), dim3(256), 0, s, j, c0, P, ldp, sP, A0, lda, sA, H, ldh, sH, E,
-                       sE, L, bad);
+// Row block j of H from Hrow (the last step of an expansion; otherwise k_cholqr
+// does it)
+template <int B>
+__global__ __launch_bounds__(256) void k_hrow(int j, int c0, const zd *__restrict__ Hrow, int64_t sR,
+                                              zd *__restrict__ H, int64_t ldh, int64_t sH) {
+  const int b = blockIdx.y, idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (j - c0) * B) return;
+  const int p = idx % B, c = c0 + idx / B;
+  H[b * sH + j + p + (int64_t)c * ldh] = Hrow[b * sR + p + (int64_t)c * B];
+}
+
+void launch_dcgs(int nb, int bq, bool fin, int j, int c0, const zd *P, int64_t ldp, int64_t sP, zd *A0, int64_t lda,
+                 int64_t sA, zd *part, zd *H, int64_t ldh, int64_t sH, zd *E, int64_t sE, zd *L, zd *Hrow, int64_t sR,
+                 int32_t *bad, hipStream_t s) {
+  const int nblk = (j + DR - 1) / DR;
+  const dim3 gp((unsigned)nblk, nb), gc((unsigned)std::max(nblk, 1), nb);
+#define EMU_DCGS(B, FIN)                                                                                            \
+  do {                                                                                                              \
+    if (nblk)                                                                                                       \
+      hipLaunchKernelGGL((k_dcgs_pre<B, FIN>), gp, dim3(256), 0, s, j, c0, P, ldp, sP, H, ldh, sH, A0, lda, sA, part); \
+    hipLaunchKernelGGL((k_dcgs_coef<B, FIN>), gc, dim3(256), 0, s, j, c0, P, ldp, sP, A0, lda, sA, part, nblk, H,   \
+                       ldh, sH, E, sE, L, Hrow, sR, bad);                                                           \
+    if (FIN && j > c0)                                                                                              \
+      hipLaunchKernelGGL(k_hrow<B>, dim3((unsigned)(((j - c0) * B + 255) / 256), nb), dim3(256), 0, s, j, c0, Hrow, \
+                         sR, H, ldh, sH);                                                                           \
+  } while (0)
+#define EMU_DCGS_B(B)           \
+  if (fin) EMU_DCGS(B, true);   \
+  else EMU_DCGS(B, false);
+  switch (bq) {
+    case 2: EMU_DCGS_B(2) break;
+    case 4: EMU_DCGS_B(4) break;
+    case 8: EMU_DCGS_B(8) break;
+    default: throw HipError("dcgs: block size must be 2, 4 or 8");
+  }
+#undef EMU_DCGS_B
+#undef EMU_DCGS
   EMU_LAUNCH_CHECK();
 }
 
-// Cholesky of the bq x bq Gram matrix G = R^H R (R upper), its inverse, and
-// Racc = R * Rprev (Rprev = identity when null).  One 64-thread workgroup per
-// instance: the matrices are loaded into LDS in parallel, one thread runs the
-// (tiny, sequential) factorisation there, and the products are written back
-// one entry per thread.  A non-positive pivot (rank-deficient block) is
-// replaced by a tiny value and counted in bad[b].
-__global__ __launch_bounds__(64) void k_cholqr(int bq, const zd *__restrict__ G, zd *__restrict__ Rinv,
-                                               const zd *__restrict__ Rprev, zd *__restrict__ Racc,
-                                               int32_t *__restrict__ bad) {
-  const int b = blockIdx.x, t = threadIdx.x;
-  const int i = t % 8, j = t / 8;
-  const bool in = i < bq && j < bq;
-  const int64_t o = (int64_t)b * bq * bq + i + j * bq;
-  __shared__ zd g[8][8], R[8][8], Ri[8][8], rp[8][8];
-  g[i][j] = in ? G[o] : zmk(0, 0);
-  rp[i][j] = (in && Rprev) ? Rprev[o] : zmk(i == j ? 1.0 : 0.0, 0);
-  R[i][j] = zmk(0, 0);
-  Ri[i][j] = zmk(0, 0);
-  __syncthreads();
-  if (t == 0) {
-    double gmax = 0;
-    for (int k = 0; k < bq; ++k) gmax = fmax(gmax, g[k][k].x);
-    for (int c = 0; c < bq; ++c) {
-      for (int r = 0; r < c; ++r) {
-        zd acc = g[r][c];
-        for (int k = 0; k < r; ++k) acc = zsub(acc, zmul(zconj(R[k][r]), R[k][c]));
-        R[r][c] = zdiv(acc, R[r][r]);
-      }
-      double d = g[c][c].x;
-      for (int k = 0; k < c; ++k) d -= R[k][c].x * R[k][c].x + R[k][c].y * R[k][c].y;
-      if (!(d > 1e-28 * gmax)) {
-        d = 1e-28 * gmax + 1e-300;
-        bad[b] += 1;
-      }
-      R[c][c] = zmk(sqrt(d), 0);
-    }
-    for (int c = 0; c < bq; ++c) {
-      Ri[c][c] = zdiv(zmk(1, 0), R[c][c]);
-      for (int r = c - 1; r >= 0; --r) {
-        zd acc = zmk(0, 0);
-        for (int k = r + 1; k <= c; ++k) acc = zadd(acc, zmul(R[r][k], Ri[k][c]));
-        Ri[r][c] = zsub(zmk(0, 0), zdiv(acc, R[r][r]));
-      }
-    }
+int64_t dcgs_part_elems(int bq, int m) { return (int64_t)((m + DR - 1) / DR) * 3 * bq * bq; }
+
+// Gram matrix of a block (n x B, ld ldw) over 256 rows per workgroup:
+// gpart[b][block][B][B], as k_combine and k_trmm_right write it
+template <int B>
+__global__ __launch_bounds__(256) void k_gram(int64_t n, const zd *__restrict__ W, int64_t ldw, int64_t sW,
+                                              zd *__restrict__ gpart) {
+  __shared__ GramLds<B> gl;
+  const int b = blockIdx.y;
+  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x, rr = r < n ? r : n - 1;
+  zd w[B];
+#pragma unroll
+  for (int q = 0; q < B; ++q) {
+    const zd v = W[b * sW + q * ldw + rr];
+    w[q] = r < n ? v : zmk(0, 0);
   }
+  const zd g = gram_thread_rows<B>(gl, w);
+  if (threadIdx.x < B * B) gpart[((int64_t)b * gridDim.x + blockIdx.x) * B * B + threadIdx.x] = g;
+}
+
+int64_t launch_gram(int nb, int64_t n, int bq, const zd *W, int64_t ldw, int64_t sW, zd *gpart, hipStream_t s) {
+  const unsigned blocks = (unsigned)((n + 255) / 256);
+  const dim3 g(blocks, nb);
+  switch (bq) {
+    case 1: hipLaunchKernelGGL(k_gram<1>, g, dim3(256), 0, s, n, W, ldw, sW, gpart); break;
+    case 2: hipLaunchKernelGGL(k_gram<2>, g, dim3(256), 0, s, n, W, ldw, sW, gpart); break;
+    case 4: hipLaunchKernelGGL(k_gram<4>, g, dim3(256), 0, s, n, W, ldw, sW, gpart); break;
+    case 8: hipLaunchKernelGGL(k_gram<8>, g, dim3(256), 0, s, n, W, ldw, sW, gpart); break;
+    default: throw HipError("gram: block size must be 1, 2, 4 or 8");
+  }
+  EMU_LAUNCH_CHECK();
+  return blocks;
+}
+
+// Cholesky-QR factor of a block from its Gram partials (gpart[b][nchunk][B][B]):
+// G = R^H R, Rinv = R^-1, Racc = R Rprev (Rprev = identity when null).  One
+// workgroup per instance: 1,024 threads add the partials, one wavefront
+// factorises.  With H the results of the block step go there as well: Racc to
+// rows j + B .. of column block j, Hrow to columns [c0, j) of row block j.
+template <int B>
+__global__ __launch_bounds__(1024) void k_cholqr(int nchunk, const zd *__restrict__ gpart, zd *__restrict__ Rinv,
+                                                 const zd *__restrict__ Rprev, zd *__restrict__ Racc, int j, int c0,
+                                                 const zd *__restrict__ Hrow, int64_t sR, zd *__restrict__ H,
+                                                 int64_t ldh, int64_t sH, int32_t *__restrict__ bad) {
+  constexpr int BB = B * B, G = 1024 / BB < 64 ? 1024 / BB : 64;
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  __shared__ zd red[G][BB], Rs[B][B], Gs[B][B];
+  if (tid < G * BB) {
+    const int o = tid % BB, g = tid / BB;
+    const zd *pp = gpart + (int64_t)b * nchunk * BB + o;
+    zd acc = zmk(0, 0);
+    for (int k = g; k < nchunk; k += 4 * G) {
+      zd v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = pp[(int64_t)min(k + u * G, nchunk - 1) * BB];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (k + u * G < nchunk) acc = zadd(acc, v[u]);
+    }
+    red[g][o] = acc;
+  }
+  if (H)
+    for (int idx = tid; idx < (j - c0) * B; idx += 1024) {
+      const int p = idx % B, c = c0 + idx / B;
+      H[b * sH + j + p + (int64_t)c * ldh] = Hrow[b * sR + p + (int64_t)c * B];
+    }
   __syncthreads();
-  if (!in) return;
-  Rinv[o] = Ri[i][j];
+  if (tid >= 64) return;
+  const int p = lane % B, q = lane / B % B;
+  zd c = zmk(0, 0);
+  if (lane < BB) {
+    for (int g = 0; g < G; ++g) c = zadd(c, red[g][lane]);
+    Gs[p][q] = c;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  double gmax = 0;
+#pragma unroll
+  for (int i = 0; i < B; ++i) gmax = fmax(gmax, Gs[i][i].x);
+  zd R, Ri;
+  const int nbad = chol_inv<B>(Gs[p][q], gmax, lane, R, Ri);
+  if (lane == 0 && nbad) bad[b] += nbad;
+  if (lane >= BB) return;
+  Rs[p][q] = R;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const int64_t o = (int64_t)b * BB;
+  Rinv[o + lane] = Ri;
   zd acc = zmk(0, 0);
-  for (int k = i; k < bq; ++k) acc = zfma(R[i][k], rp[k][j], acc);
-  Racc[o] = acc;
+#pragma unroll
+  for (int k = 0; k < B; ++k) {
+    const zd rp = Rprev ? Rprev[o + k + q * B] : zmk(k == q ? 1.0 : 0.0, 0.0);
+    if (k >= p) acc = zfma(Rs[p][k], rp, acc);
+  }
+  Racc[o + lane] = acc;
+  if (H) H[b * sH + j + B + p + (int64_t)(j + q) * ldh] = acc;
 }
 
-void launch_cholqr(int nb, int bq, const zd *G, zd *Rinv, const zd *Rprev, zd *Racc, int32_t *bad,
-                   hipStream_t s) {
-  if (bq > 8) throw HipError("cholqr: block size above 8");
-  hipLaunchKernelGGL(k_cholqr, dim3(nb), dim3(64), 0, s, bq, G, Rinv, Rprev, Racc, bad);
+void launch_cholqr(int nb, int bq, int64_t nchunk, const zd *gpart, zd *Rinv, const zd *Rprev, zd *Racc, int32_t *bad,
+                   hipStream_t s, int j, int c0, const zd *Hrow, int64_t sR, zd *H, int64_t ldh, int64_t sH) {
+#define EMU_CHOLQR(B)                                                                                               \
+  hipLaunchKernelGGL(k_cholqr<B>, dim3(nb), dim3(1024), 0, s, (int)nchunk, gpart, Rinv, Rprev, Racc, j, c0, Hrow, sR, \
+                     H, ldh, sH, bad)
+  switch (bq) {
+    case 1: EMU_CHOLQR(1); break;
+    case 2: EMU_CHOLQR(2); break;
+    case 4: EMU_CHOLQR(4); break;
+    case 8: EMU_CHOLQR(8); break;
+    default: throw HipError("cholqr: block size must be 1, 2, 4 or 8");
+  }
+#undef EMU_CHOLQR
   EMU_LAUNCH_CHECK();
 }
 
-// Wout[b][:, 0:bq] = W[b][:, 0:bq] * Rinv[b]  (bq x bq upper triangular);
-// with xi, the row-interleaved copy of Wout as well (xi[b][8 r + j], the
-// operand of the next Krylov block's SpMM, saving k_interleave8's pass)
-template <int BQ>
+// O[b][:, 0:B] = W[b][:, 0:B] * Rinv[b]  (B x B upper triangular, in place
+// allowed); with xi, the row-interleaved copy of O as well (xi[b][B r + j], the
+// operand of the next Krylov block's SpMM, saving k_interleave's pass); with
+// gpart, the Gram matrix of O over the workgroup's 256 rows
+template <int B>
 __global__ __launch_bounds__(256) void k_trmm_right(int64_t n, const zd *W, int64_t ldw, int64_t sW,
                                                     const zd *__restrict__ Ri, zd *O, int64_t ldo,
-                                                    int64_t sO, zd *__restrict__ xi) {
-  __shared__ zd rs[BQ][BQ];
+                                                    int64_t sO, zd *__restrict__ xi, zd *__restrict__ gpart) {
+  __shared__ zd rs[B][B];
+  __shared__ GramLds<B> gl;
   const int b = blockIdx.y;
-  for (int idx = threadIdx.x; idx < BQ * BQ; idx += blockDim.x) rs[idx % BQ][idx / BQ] = Ri[(int64_t)b * BQ * BQ + idx];
+  for (int idx = threadIdx.x; idx < B * B; idx += blockDim.x) rs[idx % B][idx / B] = Ri[(int64_t)b * B * B + idx];
   __syncthreads();
   const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  zd w[BQ];
+  const int64_t rr = r < n ? r : n - 1;
+  zd w[B], o[B];
 #pragma unroll
-  for (int q = 0; q < BQ; ++q) w[q] = W[b * sW + q * ldw + r];
-  zd o[BQ];
+  for (int q = 0; q < B; ++q) w[q] = W[b * sW + q * ldw + rr];
 #pragma unroll
-  for (int j = 0; j < BQ; ++j) {
+  for (int j = 0; j < B; ++j) {
     zd acc = zmk(0, 0);
 #pragma unroll
     for (int k = 0; k <= j; ++k) acc = zfma(w[k], rs[k][j], acc);
     o[j] = acc;
-    O[b * sO + j * ldo + r] = acc;
+    if (r < n) O[b * sO + j * ldo + r] = acc;
   }
-  if (xi) {
-    zd *xr = xi + (int64_t)b * BQ * n + (int64_t)BQ * r;
+  if (xi && r < n) {
+    zd *xr = xi + (int64_t)b * B * n + (int64_t)B * r;
 #pragma unroll
-    for (int j = 0; j < BQ; ++j) xr[j] = o[j];
+    for (int j = 0; j < B; ++j) xr[j] = o[j];
+  }
+  if (gpart) {
+    if (r >= n)
+#pragma unroll
+      for (int j = 0; j < B; ++j) o[j] = zmk(0, 0);
+    const zd g = gram_thread_rows<B>(gl, o);
+    if (threadIdx.x < B * B) gpart[((int64_t)b * gridDim.x + blockIdx.x) * B * B + threadIdx.x] = g;
   }
 }
 
-void launch_trmm_right(int nb, int64_t n, int bq, const zd *W, int64_t ldw, int64_t sW, const zd *Ri, zd *O,
-                       int64_t ldo, int64_t sO, hipStream_t s, zd *xi) {
-  dim3 g((unsigned)((n + 255) / 256), nb);
-  if (xi && bq != 8) throw HipError("trmm_right: the interleaved copy is for 8-column blocks");
+int64_t launch_trmm_right(int nb, int64_t n, int bq, const zd *W, int64_t ldw, int64_t sW, const zd *Ri, zd *O,
+                          int64_t ldo, int64_t sO, hipStream_t s, zd *xi, zd *gpart) {
+  const unsigned blocks = (unsigned)((n + 255) / 256);
+  dim3 g(blocks, nb);
+#define EMU_TRMM(B) hipLaunchKernelGGL(k_trmm_right<B>, g, dim3(256), 0, s, n, W, ldw, sW, Ri, O, ldo, sO, xi, gpart)
   switch (bq) {
-    case 1: hipLaunchKernelGGL(k_trmm_right<1>, g, dim3(256), 0, s, n, W, ldw, sW, Ri, O, ldo, sO, nullptr); break;
-    case 2: hipLaunchKernelGGL(k_trmm_right<2>, g, dim3(256), 0, s, n, W, ldw, sW, Ri, O, ldo, sO, nullptr); break;
-    case 4: hipLaunchKernelGGL(k_trmm_right<4>, g, dim3(256), 0, s, n, W, ldw, sW, Ri, O, ldo, sO, nullptr); break;
-    case 8: hipLaunchKernelGGL(k_trmm_right<8>, g, dim3(256), 0, s, n, W, ldw, sW, Ri, O, ldo, sO, xi); break;
+    case 1: EMU_TRMM(1); break;
+    case 2: EMU_TRMM(2); break;
+    case 4: EMU_TRMM(4); break;
+    case 8: EMU_TRMM(8); break;
     default: throw HipError("trmm_right: block size must be 1, 2, 4 or 8");
   }
+#undef EMU_TRMM
   EMU_LAUNCH_CHECK();
+  return blocks;
 }
 
 // Dst[b][i + j*ldd] (+)= Src[b][i + j*lds] for i < rows, j < cols
