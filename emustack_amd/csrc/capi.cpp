@@ -221,7 +221,7 @@ static int modes2d_impl(emu_ctx *ctx, emu_mesh *mesh, int64_t nbatch, const doub
     if (a.precision != 0 && a.precision != 1) return fail(EMU_E_ARG, "precision must be 0 (FP64) or 1 (mixed)");
     if (opts && opts[2] > 0) a.block = (int64_t)opts[2];
     if (opts && opts[3] > 0) a.ncv = (int64_t)opts[3];
-    if (a.block != 1 && a.block != 2 && a.block != 4 && a.block != 8)
+    if (a.block != 0 && a.block != 1 && a.block != 2 && a.block != 4 && a.block != 8)
       return fail(EMU_E_ARG, "Krylov block size must be 1, 2, 4 or 8");
     a.beta = beta1;
     a.J = overlap_J;

@@ -704,6 +704,12 @@ static bool ks_project(KSState &st, int m, int bq, int nev, int keep, double tol
   return conv;
 }
 
+// Columns kept at a restart; m minus it is a multiple of the block size.
+static int restart_size(int m, int bq, int nev) {
+  const int keep = std::min(m - bq, nev + (m - nev) / 2);
+  return m - ((m - keep + bq - 1) / bq) * bq;
+}
+
 struct EigResult {
   std::vector<cplx> mu;  // nb x nev
   int64_t ops = 0, restarts = 0, steps = 0, rank_fixes = 0;
@@ -860,8 +866,7 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
   res.mu.assign((size_t)nb * nev, 0);
   std::vector<int> schur_na;  // active Schur sizes, recorded when the stage timer is on
   int k = 0;
-  int keep = std::min(m - bq, nev + (m - nev) / 2);
-  keep = m - ((m - keep + bq - 1) / bq) * bq;  // (m - keep) multiple of bq
+  const int keep = restart_size(m, bq, nev);
   if (keep < nev) throw std::invalid_argument("Krylov subspace too small for num_BMs");
   std::vector<zd> Hh((size_t)nb * sH);
   std::vector<std::vector<cplx>> ritz(nb);
@@ -1427,10 +1432,22 @@ void calc_modes(Ctx *c, DevMesh &dm, const ModesArgs &a) {
   if (nl < 1 || nval < 1 || ntyp < dm.ntyp) throw std::invalid_argument("calc_modes: bad sizes");
   // Krylov dimension: ARPACK's nvect = 2 nval + nval/2 + 3 (py_calc_modes.f:256),
   // rounded up to a whole number of blocks
-  const int bq = (int)a.block;
+  // Block size, when the caller names none.  Narrower blocks reach a higher
+  // polynomial degree in the same m vectors, so they need fewer restarts and
+  // projected Schur problems; wider ones share each pass over the factors
+  // among more columns.  Whole solves with blocks of 8 / 4 / 2, ms: n = 2 k
+  // unknowns, 1 light 94 / 68 / 60, 8 lights 159 / 112 / 96; 6 k, 2 lights
+  // 202 / 149 / 146; 32 k, 1 light 662 / 563 / 672, 4 lights 1042 / 978 / 1360.
+  // Calls that fill the card by themselves (8 lights at 32 k: 16 factors) keep
+  // 8: four such calls at once are bound by the factors' bytes and solve 3.15
+  // wavelengths per second with 8 columns, 2.82 with 4.
+  // The dimension and what it is refused for are those of 8-column blocks.
+  const int bq = a.block > 0 ? (int)a.block : (int64_t)nb * n < 400000 ? 4 : 8;
+  const int wide = a.block > 0 ? bq : 8;
   int m = a.ncv > 0 ? (int)a.ncv : 2 * nval + nval / 2 + 3;
-  m = ((m + bq - 1) / bq) * bq;
-  if (m + bq >= n || nval >= m) throw std::invalid_argument("calc_modes: num_BMs too large for the mesh");
+  m = ((m + wide - 1) / wide) * wide;
+  if (m + wide >= n || nval >= m) throw std::invalid_argument("calc_modes: num_BMs too large for the mesh");
+  if (restart_size(m, wide, nval) < nval) throw std::invalid_argument("Krylov subspace too small for num_BMs");
   std::vector<cplx> pp, qq, sh;
   std::vector<double> bl, k0;
   instance_params(a, (int)a.eh, pp, qq, sh, bl, k0);

@@ -46,7 +46,7 @@ struct ModesArgs {
   const double *bloch = nullptr;   // nl x 2
   const double *shift = nullptr;   // nl complex
   double tol = 1e-12;  // relative residual of every wanted Ritz pair (see ks_project)
-  int64_t block = 8;               // Krylov block size (1, 2, 4 or 8)
+  int64_t block = 0;               // Krylov block size (1, 2, 4 or 8; 0: by the size of the call)
   // 0: complex128 everywhere; 1: mixed: the Krylov solves read a complex64
   // copy of the (FP64-computed) inverted factor, and every converged pair's
   // beta is corrected by the FP64 two-sided Rayleigh quotient of the pencil

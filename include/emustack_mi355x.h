@@ -132,8 +132,9 @@ int emu_calc_modes_2d_fields(emu_ctx *ctx, emu_mesh *mesh, double lambda, int64_
  * read a complex64 copy of the FP64 inverted factor, and each converged
  * pair's beta is the FP64 two-sided Rayleigh quotient of the pencil);
  * opts[2] = Krylov
- * block size (1, 2, 4 or 8; <= 0: default 8); opts[3] = Krylov dimension
- * (<= 0: the reference's 2 nval + nval/2 + 3, rounded up to whole blocks).  stats[0..7] (may be NULL): OP applications,
+ * block size (1, 2, 4 or 8; <= 0: 4, or 8 where 2 nbatch neq >= 400000); opts[3] = Krylov dimension
+ * (<= 0: the reference's 2 nval + nval/2 + 3, rounded up to whole blocks, or
+ * to a multiple of 8 where opts[2] names no block size).  stats[0..7] (may be NULL): OP applications,
  * restarts (max over instances), pivot perturbations, Arnoldi steps,
  * rank repairs, modes whose beta came from the FP64 two-sided Rayleigh
  * quotient, modes that kept the Ritz value (quotient disagreed by > 1e-4),
@@ -272,10 +273,10 @@ int emu_film_modes_batch(emu_ctx *ctx, int64_t nbatch, int64_t npw, const double
  * solve sweep; enable = 0 stops.  out[k*3 + {0,1,2}] (may be NULL) for kernel
  * class k: launches timed, total milliseconds, total algorithmic bytes of
  * those launches.  Classes: 0 forward-solve level sweep (k_fwd), 1 backward
- * level sweep (k_bwd), 2 Gram-Schmidt projections (k_atb_mfma16 for the
- * 8-column blocks, k_atb_tall for smaller ones), 3 Gram-Schmidt updates
- * (k_combine; k_sub_vh_blk for blocks below 8 columns), 4 mass-matrix
- * product of the Krylov block (k_spmm_il; k_spmm below 8 columns),
+ * level sweep (k_bwd), 2 Gram-Schmidt projections (k_atb_mfma16 for
+ * blocks of columns, k_atb_tall for single vectors), 3 Gram-Schmidt updates
+ * (k_combine; k_sub_vh_blk for single vectors), 4 mass-matrix
+ * product of the Krylov block (k_spmm_il; k_spmm for single vectors),
  * 5..7 reserved. */
 int emu_profile(emu_ctx *ctx, int enable, int every, double *out);
 
