@@ -192,17 +192,16 @@ __device__ __forceinline__ double wave_max(double v) {
                           __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
 
-// 1 / d by one reciprocal of |d|^2, scaled by the larger part's exponent
-// (v_rcp_f64 and two Newton steps: within 2 ulp; no overflow for any normal
-// d).  Smith's division takes three dependent divides.
+// 1 / d, Smith's division without its branch: the bits of zdiv(1, d), which the
+// update rows and k_panel use.  (One reciprocal of |d|^2 is a shorter chain by
+// 1 to 2 % of a panel, but its other rounding decides near ties of the pivot
+// search differently, and with them the rounding of the complex64 factor.)
 __device__ __forceinline__ zd zrecip(zd d) {
-  const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(d.x), fabs(d.y)));
-  const double x = __builtin_amdgcn_ldexp(d.x, -e), y = __builtin_amdgcn_ldexp(d.y, -e);
-  const double n = fma(x, x, y * y);
-  double r = __builtin_amdgcn_rcp(n);
-  r = fma(r, fma(-n, r, 1.0), r);
-  r = fma(r, fma(-n, r, 1.0), r);
-  return zmk(__builtin_amdgcn_ldexp(x * r, -e), __builtin_amdgcn_ldexp(-y * r, -e));
+  const bool xl = fabs(d.x) >= fabs(d.y);
+  const double p = xl ? d.x : d.y, q = xl ? d.y : d.x;
+  const double r = q / p, den = p + q * r;
+  const double u = 1.0 / den, v = r / den;
+  return xl ? zmk(u, -v) : zmk(v, -u);
 }
 
 // Panel step with the panel in registers (up to 64 NW RPT pivot-candidate
@@ -228,7 +227,7 @@ __device__ __forceinline__ zd zrecip(zd d) {
 // k_panel_apply, which moves the other columns' entries in one gather instead
 // of up to 32 dependent swaps.
 // Measured, mean per launch (k_panel in brackets): the dense LUs of a 64-point
-// 200-mode cascade 43 us (85), the 8,000-triangle mesh with 2 instances 60 us
+// 200-mode cascade 44 us (85), the 8,000-triangle mesh with 2 instances 61 us
 // (164).
 template <int NW, int RPT, int CW>
 __global__ __launch_bounds__(64 * NW) void k_panel_reg(const int32_t *__restrict__ tasks, int k0, FrontArrays A,
