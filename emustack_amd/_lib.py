@@ -35,12 +35,14 @@ c_i32p = ctypes.POINTER(ctypes.c_int32)
 c_vp = ctypes.c_void_p
 
 EXPORTS = [
-    'emu_last_error', 'emu_ctx_create', 'emu_ctx_destroy', 'emu_set_lapack', 'emu_mesh_load',
+    'emu_last_error', 'emu_ctx_create', 'emu_ctx_destroy', 'emu_set_lapack', 'emu_set_lapack_hessenberg',
+    'emu_mesh_load',
     'emu_mesh_analyze', 'emu_mesh_symbolic', 'emu_mesh_free', 'emu_mesh_info', 'emu_mesh_arrays',
     'emu_mesh_geometry', 'emu_calc_modes_2d', 'emu_calc_modes_2d_batch', 'emu_assemble', 'emu_lu_solve',
     'emu_profile', 'emu_mesh_create_1d', 'emu_calc_modes_1d', 'emu_calc_modes_1d_batch', 'emu_star_cascade_batch',
     'emu_material_index', 'emu_assemble_noalloc', 'emu_calc_modes_2d_fields', 'emu_calc_modes_1d_fields',
     'emu_calc_modes_2d_submit', 'emu_job_wait', 'emu_film_modes_batch',
+    'emu_schur',
 ]
 
 
@@ -87,8 +89,9 @@ def _host_lapack_threads(nl):
 
 
 def _lapack_pointers():
-    """Addresses of zgees/ztrsen/ztrevc from scipy's LAPACK build (used for
-    the small projected Schur problem of the eigensolver, on the host)."""
+    """Addresses of zgees/ztrsen/ztrevc and zgehrd/zunghr from scipy's LAPACK
+    build (used for the small projected Schur problem of the eigensolver, on
+    the host)."""
     import scipy.linalg.cython_lapack as cl
     get_name = ctypes.pythonapi.PyCapsule_GetName
     get_name.restype = ctypes.c_char_p
@@ -97,7 +100,7 @@ def _lapack_pointers():
     get_ptr.restype = ctypes.c_void_p
     get_ptr.argtypes = [ctypes.py_object, ctypes.c_char_p]
     out = []
-    for name in ('zgees', 'ztrsen', 'ztrevc'):
+    for name in ('zgees', 'ztrsen', 'ztrevc', 'zgehrd', 'zunghr'):
         cap = cl.__pyx_capi__[name]
         out.append(get_ptr(cap, get_name(cap)))
     return out
@@ -118,6 +121,8 @@ def lib():
         L.emu_ctx_destroy.argtypes = [c_vp]
         L.emu_ctx_destroy.restype = None
         L.emu_set_lapack.argtypes = [c_vp, c_vp, c_vp]
+        L.emu_set_lapack_hessenberg.argtypes = [c_vp, c_vp]
+        L.emu_schur.argtypes = [c_i64, c_dp, c_i32p, c_dp, c_dp]
         L.emu_mesh_load.argtypes = [c_vp, ctypes.c_char_p, ctypes.c_int, ctypes.POINTER(c_vp)]
         L.emu_mesh_analyze.argtypes = [ctypes.c_char_p, ctypes.c_int, ctypes.POINTER(c_vp)]
         L.emu_mesh_symbolic.argtypes = [c_vp, c_i32p, c_i64p, c_i64p, c_i32p, c_i32p, c_i64p]
@@ -158,7 +163,8 @@ def lib():
                                                c_dp, c_dp, c_dp, c_dp, c_dp, c_dp]
         for f in EXPORTS:
             getattr(L, f)
-        rc = L.emu_set_lapack(*_lapack_pointers())
+        ptrs = _lapack_pointers()
+        rc = L.emu_set_lapack(*ptrs[:3]) or L.emu_set_lapack_hessenberg(*ptrs[3:])
         if rc != EMU_OK:
             raise EmuError(rc, L.emu_last_error().decode())
         _lib = L

@@ -129,6 +129,21 @@ int emu_set_lapack(void *zgees, void *ztrsen, void *ztrevc) {
   return EMU_OK;
 }
 
+int emu_set_lapack_hessenberg(void *zgehrd, void *zunghr) {
+  if (!zgehrd || !zunghr) return fail(EMU_E_ARG, "emu_set_lapack_hessenberg: NULL routine");
+  emu::set_lapack_hessenberg(zgehrd, zunghr);
+  return EMU_OK;
+}
+
+int emu_schur(int64_t n, const double *a, const int32_t *select, double *t, double *q) {
+  if (n < 1 || n > 8192 || !a || !select || !t || !q) return fail(EMU_E_ARG, "emu_schur: bad argument");
+  EMU_GUARD({
+    std::vector<int> sel(select, select + n);
+    emu::schur((int)n, reinterpret_cast<const std::complex<double> *>(a), sel.data(),
+               reinterpret_cast<std::complex<double> *>(t), reinterpret_cast<std::complex<double> *>(q));
+  })
+}
+
 int emu_mesh_load(emu_ctx *ctx, const char *path, int leaf_size, emu_mesh **out) {
   if (!ctx || !path || !out) return fail(EMU_E_ARG, "emu_mesh_load: NULL argument");
   EMU_GUARD({

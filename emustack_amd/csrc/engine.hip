@@ -20,6 +20,7 @@
 
 #include "emu_host.h"
 #include "engine.h"
+#include "schur.h"
 #include "fem_basis.h"
 #include "engine_api.h"
 
@@ -44,7 +45,9 @@ typedef void (*ztrsen_t)(char *, char *, int *, int *, cplx *, int *, cplx *, in
                          double *, cplx *, int *, int *);
 typedef void (*ztrevc_t)(char *, char *, int *, int *, cplx *, int *, cplx *, int *, cplx *, int *, int *, int *,
                          cplx *, double *, int *);
+typedef void (*zgehrd_t)(int *, int *, int *, cplx *, int *, cplx *, cplx *, int *, int *);
 static zgees_t g_zgees = nullptr;
+static zgehrd_t g_zgehrd = nullptr, g_zunghr = nullptr;  // zunghr takes the same arguments
 static ztrsen_t g_ztrsen = nullptr;
 static ztrevc_t g_ztrevc = nullptr;
 
@@ -52,6 +55,10 @@ void set_lapack(void *a, void *b, void *c) {
   g_zgees = (zgees_t)a;
   g_ztrsen = (ztrsen_t)b;
   g_ztrevc = (ztrevc_t)c;
+}
+void set_lapack_hessenberg(void *a, void *b) {
+  g_zgehrd = (zgehrd_t)a;
+  g_zunghr = (zgehrd_t)b;
 }
 static int dummy_select(cplx *) { return 0; }
 bool lapack_ready() { return g_zgees && g_ztrsen && g_ztrevc; }
@@ -568,6 +575,80 @@ static void ks_restart_blocks(KSState &S, int m, int bq, int keep, int ld, int64
   }
 }
 
+// A = Q T Q^H (A: n x n, leading dimension ld; T, Q: n x n).  Hessenberg
+// reduction and schur_hessenberg; zgees where the CPU lacks its instructions,
+// where it gave up, and for magnitudes whose squares leave the range.  zgees
+// spends most of its time on scalar rotations: 4.3 against 1.2 ms at n = 90,
+// 14.4 against 5.7 at 176, 117 against 58 at 440 (one core).
+// The reduction is LAPACK's from 192 rows on, where its blocks keep the matrix
+// out of the third-level cache (440 rows: 66 against 107 ms for schur_reduce on
+// a slower machine); below, its many small BLAS calls wait for each other in
+// the library's allocator (90 rows, 16 threads: 1.8 ms, alone 0.43).
+static void schur_form(int n, const cplx *A, int ld, cplx *T, cplx *Q) {
+  double top = 0;
+  auto copy_in = [&]() {
+    for (int j = 0; j < n; ++j) std::copy(A + (size_t)j * ld, A + (size_t)j * ld + n, T + (size_t)j * n);
+  };
+  copy_in();
+  for (size_t i = 0; i < (size_t)n * n; ++i)
+    top = std::max(top, std::max(std::fabs(T[i].real()), std::fabs(T[i].imag())));
+  int lda = n, lwork = -1, info = 0;
+  cplx wq;
+  std::vector<cplx> work;
+  if (schur_available() && top > 1e-100 && top < 1e100) {
+    if (n < 192 || !g_zgehrd) {
+      schur_reduce(n, T, n, Q, n);
+    } else {
+      int ilo = 1, ihi = n;
+      std::vector<cplx> tau(n);
+      g_zgehrd(&n, &ilo, &ihi, T, &lda, tau.data(), &wq, &lwork, &info);
+      lwork = std::max(64 * n, (int)wq.real());  // zunghr asks for no more
+      work.resize(lwork);
+      g_zgehrd(&n, &ilo, &ihi, T, &lda, tau.data(), work.data(), &lwork, &info);
+      std::copy(T, T + (size_t)n * n, Q);
+      if (info == 0) g_zunghr(&n, &ilo, &ihi, Q, &lda, tau.data(), work.data(), &lwork, &info);
+      for (int j = 0; j + 2 < n; ++j) std::fill(T + j + 2 + (size_t)j * n, T + (size_t)(j + 1) * n, cplx(0));
+    }
+    if (info == 0 && schur_hessenberg(n, T, n, Q, n, n)) return;
+    copy_in();
+    lwork = -1;
+  }
+  char jobvs = 'V', sort = 'N';
+  int sdim = 0;
+  std::vector<cplx> w(n);
+  std::vector<double> rwork(n);
+  std::vector<int> bwork(n);
+  g_zgees(&jobvs, &sort, dummy_select, &n, T, &lda, &sdim, w.data(), Q, &lda, &wq, &lwork, rwork.data(), bwork.data(),
+          &info);
+  lwork = std::max(1, (int)wq.real());
+  work.resize(std::max((int)work.size(), lwork));
+  g_zgees(&jobvs, &sort, dummy_select, &n, T, &lda, &sdim, w.data(), Q, &lda, work.data(), &lwork, rwork.data(),
+          bwork.data(), &info);
+  if (info != 0) throw std::runtime_error("zgees failed, info=" + std::to_string(info));
+}
+
+// The selected rows of T first, in their order (T, Q: n x n).  ztrsen meets
+// every exchange with strided row rotations: 0.63 -> 0.13 ms at n = 90, 23 -> 3.4
+// at 440 for the two selections of a restart.
+static void schur_select(int n, cplx *T, cplx *Q, int *sel) {
+  if (schur_available()) {
+    schur_reorder(n, T, n, Q, n, n, sel);
+    return;
+  }
+  char job = 'N', compq = 'V';
+  int mm = 0, lw = std::max(1, n), inf = 0;
+  double sv = 0, sep = 0;
+  std::vector<cplx> wk(lw), w(n);
+  g_ztrsen(&job, &compq, sel, &n, T, &n, Q, &n, w.data(), &mm, &sv, &sep, wk.data(), &lw, &inf);
+  if (inf != 0) throw std::runtime_error("ztrsen failed, info=" + std::to_string(inf));
+}
+
+void schur(int n, const cplx *A, int *sel, cplx *T, cplx *Q) {
+  if (!lapack_ready()) throw LapackMissing("host LAPACK routines not registered (emu_set_lapack)");
+  schur_form(n, A, n, T, Q);
+  schur_select(n, T, Q, sel);
+}
+
 // Schur-decompose H[:m,:m], order the `keep` largest |theta| first and the
 // `nev` largest among them first of all, test the residuals
 // ||B Q y_i|| <= tol max(eps^(2/3), |theta_i|) of the leading nev Ritz pairs (B = last bq rows
@@ -590,21 +671,7 @@ static bool ks_project(KSState &st, int m, int bq, int nev, int keep, double tol
   const int ld = m + bq;
   const int a0 = std::min(st.nlock, nev), na = m - a0;
   std::vector<cplx> TA((size_t)na * na), QA((size_t)na * na);
-  for (int j = 0; j < na; ++j)
-    for (int i = 0; i < na; ++i) TA[i + (size_t)j * na] = st.H[(a0 + i) + (size_t)(a0 + j) * ld];
-  std::vector<cplx> thA(na);
-  int n = na, lda = na, sdim = 0, ldvs = na, info = 0, lwork = -1;
-  char jobvs = 'V', sort = 'N';
-  std::vector<double> rwork(na);
-  std::vector<int> bwork(na);
-  cplx wq;
-  g_zgees(&jobvs, &sort, dummy_select, &n, TA.data(), &lda, &sdim, thA.data(), QA.data(), &ldvs, &wq, &lwork,
-          rwork.data(), bwork.data(), &info);
-  lwork = std::max(1, (int)wq.real());
-  std::vector<cplx> work(lwork);
-  g_zgees(&jobvs, &sort, dummy_select, &n, TA.data(), &lda, &sdim, thA.data(), QA.data(), &ldvs, work.data(),
-          &lwork, rwork.data(), bwork.data(), &info);
-  if (info != 0) throw std::runtime_error("zgees failed, info=" + std::to_string(info));
+  schur_form(na, &st.H[a0 + (size_t)a0 * ld], ld, TA.data(), QA.data());
   st.T.assign((size_t)m * m, 0);
   st.Q.assign((size_t)m * m, 0);
   for (int j = 0; j < a0; ++j) {
@@ -626,9 +693,6 @@ static bool ks_project(KSState &st, int m, int bq, int nev, int keep, double tol
   }
   st.theta.assign(m, 0);
   for (int i = 0; i < m; ++i) st.theta[i] = st.T[i + (size_t)i * m];
-  n = m;
-  lda = m;
-  ldvs = m;
   auto reorder = [&](int count) {
     // locked columns stay selected (and first); the rest by largest |theta|
     std::vector<int> idx(na);
@@ -638,15 +702,8 @@ static bool ks_project(KSState &st, int m, int bq, int nev, int keep, double tol
     std::vector<int> sel(m, 0);
     for (int i = 0; i < a0; ++i) sel[i] = 1;
     for (int i = 0; i < count - a0; ++i) sel[idx[i]] = 1;
-    char job = 'N', compq = 'V';
-    int mm = 0, lw = std::max(1, m), inf = 0;
-    double sv = 0, sep = 0;
-    std::vector<cplx> wk(lw);
-    std::vector<cplx> w(m);
-    g_ztrsen(&job, &compq, sel.data(), &n, st.T.data(), &lda, st.Q.data(), &ldvs, w.data(), &mm, &sv, &sep,
-             wk.data(), &lw, &inf);
-    if (inf != 0) throw std::runtime_error("ztrsen failed, info=" + std::to_string(inf));
-    st.theta = w;
+    schur_select(m, st.T.data(), st.Q.data(), sel.data());
+    for (int i = 0; i < m; ++i) st.theta[i] = st.T[i + (size_t)i * m];
   };
   reorder(keep);
   reorder(nev);
@@ -1439,7 +1496,7 @@ void calc_modes(Ctx *c, DevMesh &dm, const ModesArgs &a) {
   // unknowns, 1 light 94 / 68 / 60, 8 lights 159 / 112 / 96; 6 k, 2 lights
   // 202 / 149 / 146; 32 k, 1 light 662 / 563 / 672, 4 lights 1042 / 978 / 1360.
   // Calls that fill the card by themselves (8 lights at 32 k: 16 factors) keep
-  // 8: four such calls at once are bound by the factors' bytes and solve 3.15
+  // 8: four such calls at once are bound by the factors' bytes and solve 3.27
   // wavelengths per second with 8 columns, 2.82 with 4.
   // The dimension and what it is refused for are those of 8-column blocks.
   const int bq = a.block > 0 ? (int)a.block : (int64_t)nb * n < 400000 ? 4 : 8;

@@ -1,5 +1,6 @@
 // Internal interface between the C-ABI layer (capi.cpp) and the engine.
 #pragma once
+#include <complex>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -20,7 +21,10 @@ struct LapackMissing : std::runtime_error {
 };
 
 void set_lapack(void *zgees, void *ztrsen, void *ztrevc);
+void set_lapack_hessenberg(void *zgehrd, void *zunghr);
 bool lapack_ready();
+// A = Q T Q^H (column-major n x n), the rows with sel != 0 of T first
+void schur(int n, const std::complex<double> *A, int *sel, std::complex<double> *T, std::complex<double> *Q);
 Ctx *ctx_create(int device);
 void ctx_destroy(Ctx *c);
 void profile(Ctx *c, int enable, int every, double *out);

@@ -50,6 +50,10 @@ void emu_ctx_destroy(emu_ctx *ctx);
  * role zlahqr/ztrevc play inside ARPACK (zarpack.f:3960 zneigh).  Must be set
  * once per process before the first eigensolve. */
 int emu_set_lapack(void *zgees, void *ztrsen, void *ztrevc);
+/* Optional: zgehrd and zunghr.  CPUs with AVX-512 bring the projected problem
+ * to Schur form by the library's own QR iteration (others by zgees); large
+ * ones reach Hessenberg form faster through these two. */
+int emu_set_lapack_hessenberg(void *zgehrd, void *zunghr);
 
 /* Load a .mail mesh: topology, DOF numbering, periodic merge, sparse
  * pattern (py_calc_modes.f:297-522), nested-dissection symbolic LU analysis
@@ -281,6 +285,10 @@ int emu_film_modes_batch(emu_ctx *ctx, int64_t nbatch, int64_t npw, const double
 int emu_profile(emu_ctx *ctx, int enable, int every, double *out);
 
 /* Stage entry points (parity tests and benchmarks). */
+
+/* Schur form A = Q T Q^H of a projected matrix on the host (n x n complex,
+ * column-major), the eigenvalues with select != 0 moved to the top of T. */
+int emu_schur(int64_t n, const double *a, const int32_t *select, double *t, double *q);
 
 /* Assembly of mat1 = K - shift*M and mat2 = M (asmbly.f:3-341) for nbatch
  * instances: pp, qq [nbatch*2*nb_typ_el], shift [nbatch*2], bloch [nbatch*2].
