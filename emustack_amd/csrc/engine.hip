@@ -1491,11 +1491,12 @@ void calc_modes(Ctx *c, DevMesh &dm, const ModesArgs &a) {
   // rounded up to a whole number of blocks
   // Block size, when the caller names none.  Narrower blocks reach a higher
   // polynomial degree in the same m vectors, so they need fewer restarts and
-  // projected Schur problems; wider ones share each pass over the factors
-  // among more columns.  Whole solves with blocks of 8 / 4 / 2, ms: n = 2 k
-  // unknowns, 1 light 94 / 68 / 60, 8 lights 159 / 112 / 96; 6 k, 2 lights
-  // 202 / 149 / 146; 32 k, 1 light 662 / 563 / 672, 4 lights 1042 / 978 / 1360.
-  // Calls that fill the card by themselves (8 lights at 32 k: 16 factors) keep
+  // projected Schur problems; wider ones share each pass over the factors and
+  // the basis among more columns.  Whole solves with blocks of 8 / 4 / 2, ms:
+  // n = 6 k unknowns, 1 light 46 / 40 / 40, 8 lights 86 / 68 / 67; 18 k, 2
+  // lights 118 / 100 / 106, 8 lights 260 / 192 / 239; 96 k, 1 light 404 / 383 /
+  // 522, 4 lights 808 / 803 / 1209.
+  // Calls that fill the card by themselves (8 lights at 96 k: 16 factors) keep
   // 8: four such calls at once are bound by the factors' bytes and solve 3.27
   // wavelengths per second with 8 columns, 2.82 with 4.
   // The dimension and what it is refused for are those of 8-column blocks.
