@@ -42,7 +42,7 @@ EXPORTS = [
     'emu_profile', 'emu_mesh_create_1d', 'emu_calc_modes_1d', 'emu_calc_modes_1d_batch', 'emu_star_cascade_batch',
     'emu_material_index', 'emu_assemble_noalloc', 'emu_calc_modes_2d_fields', 'emu_calc_modes_1d_fields',
     'emu_calc_modes_2d_submit', 'emu_job_wait', 'emu_film_modes_batch',
-    'emu_schur',
+    'emu_schur', 'emu_star_cascade_rows',
 ]
 
 
@@ -146,6 +146,8 @@ def lib():
         c_dpp = ctypes.POINTER(c_dp)
         L.emu_star_cascade_batch.argtypes = [c_vp, c_i64, c_i64, c_i64, c_i64p, c_i64p, c_dpp, c_dpp, c_dpp, c_dpp,
                                              c_dp, c_dp, c_dp, c_i64p, c_dp, c_dp, c_dp, c_dp, c_dp]
+        L.emu_star_cascade_rows.argtypes = (L.emu_star_cascade_batch.argtypes[:10] + [c_i64p] +
+                                            L.emu_star_cascade_batch.argtypes[10:])
         L.emu_calc_modes_1d_batch.argtypes = [c_vp, c_vp, c_i64, c_dp, c_i64, c_i64, c_i64, c_dp, c_dp, c_dp,
                                               c_i64, c_i64, c_i64, c_i64, c_dp, c_dp, c_dp, c_dp, c_dp, c_dp,
                                               c_i64p]
@@ -392,17 +394,19 @@ class Context:
             keep.append(a)
             return a.view(np.float64).ctypes.data_as(c_dp)
 
-        def fptr(a):  # (nb, r, c) -> per point F-order
+        rows = np.zeros((L, 2), np.int64)
+
+        def mptr(a, l, k):  # (nb, r, c) matrices, row- or column-major as they are
             if a is None:
                 return None
-            a = np.ascontiguousarray(np.asarray(a, np.complex128).transpose(0, 2, 1))
-            keep.append(a)
-            return a.view(np.float64).ctypes.data_as(c_dp)
+            a = np.asarray(a, np.complex128)
+            rows[l, k] = not a.transpose(0, 2, 1).flags.c_contiguous
+            return cptr(a if rows[l, k] else a.transpose(0, 2, 1))
         arr = lambda xs: (c_dp * L)(*xs)
         kz_p = arr([cptr(k) for k in kz])
         Z_p = arr([cptr(z) for z in Z])
-        J_p = arr([fptr(j) for j in J])
-        Jd_p = arr([fptr(j) for j in Jd])
+        J_p = arr([mptr(j, l, 0) for l, j in enumerate(J)])
+        Jd_p = arr([mptr(j, l, 1) for l, j in enumerate(Jd)])
         kinds = np.asarray(kinds, np.int64)
         nmodes = np.array([np.asarray(k).shape[1] for k in kz], np.int64)
         heights = np.asarray(heights, np.float64)
@@ -417,9 +421,9 @@ class Context:
         t_l = np.zeros((nb, L - 1))
         R = np.zeros((nb, d, d), np.complex128) if want_nets else None
         T = np.zeros((nb, d, d), np.complex128) if want_nets else None
-        check(lib().emu_star_cascade_batch(self.h, nb, L, d // 2, ptr(kinds, c_i64p), ptr(nmodes, c_i64p), kz_p,
-                                           Z_p, J_p, Jd_p, ptr(heights), cptr(Zair), cptr(d_minus),
-                                           ptr(nprop, c_i64p), ptr(R.view(np.float64)) if want_nets else None,
+        check(lib().emu_star_cascade_rows(self.h, nb, L, d // 2, ptr(kinds, c_i64p), ptr(nmodes, c_i64p), kz_p,
+                                          Z_p, J_p, Jd_p, ptr(rows, c_i64p), ptr(heights), cptr(Zair), cptr(d_minus),
+                                          ptr(nprop, c_i64p), ptr(R.view(np.float64)) if want_nets else None,
                                            ptr(T.view(np.float64)) if want_nets else None, ptr(a_l), ptr(r_l),
                                            ptr(t_l)))
         if want_nets:  # stored per point column-major

@@ -439,7 +439,7 @@ int emu_calc_modes_1d_fields(emu_ctx *ctx, emu_mesh *mesh, double lambda, int64_
                       nullptr, sol_P2);
 }
 
-int emu_star_cascade_batch(emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_t neq_PW, const int64_t *kind,
+static int star_cascade_call(const int64_t *rows, emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_t neq_PW, const int64_t *kind,
                            const int64_t *nmodes, const double *const *kz, const double *const *Z,
                            const double *const *J, const double *const *J_dagger, const double *heights,
                            const double *Zair, const double *d_minus, const int64_t *nprop, double *R_net,
@@ -466,6 +466,7 @@ int emu_star_cascade_batch(emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_
     a.Z = Z;
     a.J = J;
     a.Jd = J_dagger;
+    a.rows = rows;
     a.heights = heights;
     a.Zair = Zair;
     a.d_minus = d_minus;
@@ -477,6 +478,24 @@ int emu_star_cascade_batch(emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_
     a.t_list = t_list;
     emu::star_cascade(ctx->c, a);
   })
+}
+
+int emu_star_cascade_batch(emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_t neq_PW, const int64_t *kind,
+                           const int64_t *nmodes, const double *const *kz, const double *const *Z,
+                           const double *const *J, const double *const *J_dagger, const double *heights,
+                           const double *Zair, const double *d_minus, const int64_t *nprop, double *R_net,
+                           double *T_net, double *a_list, double *r_list, double *t_list) {
+  return star_cascade_call(nullptr, ctx, nbatch, nlayers, neq_PW, kind, nmodes, kz, Z, J, J_dagger, heights, Zair, d_minus, nprop, R_net,
+                           T_net, a_list, r_list, t_list);
+}
+
+int emu_star_cascade_rows(emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_t neq_PW, const int64_t *kind,
+                           const int64_t *nmodes, const double *const *kz, const double *const *Z,
+                           const double *const *J, const double *const *J_dagger, const int64_t *row_major, const double *heights,
+                           const double *Zair, const double *d_minus, const int64_t *nprop, double *R_net,
+                           double *T_net, double *a_list, double *r_list, double *t_list) {
+  return star_cascade_call(row_major, ctx, nbatch, nlayers, neq_PW, kind, nmodes, kz, Z, J, J_dagger, heights, Zair, d_minus, nprop, R_net,
+                           T_net, a_list, r_list, t_list);
 }
 
 int emu_material_index(emu_ctx *ctx, int64_t nmat, const int64_t *kind, const int64_t *offset,

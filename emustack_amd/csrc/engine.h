@@ -223,6 +223,7 @@ struct DevMesh {
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
+  hipStream_t upload = nullptr;  // large uploads beside the stream's kernels (created on first use)
   Profiler prof;
   std::vector<void *> bufs;
   std::vector<size_t> sizes;
@@ -254,6 +255,7 @@ struct Ctx {
   ~Ctx() {
     for (auto &kv : dense) delete kv.second;
     for (void *p : bufs) (void)hipFree(p);
+    if (upload) (void)hipStreamDestroy(upload);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };

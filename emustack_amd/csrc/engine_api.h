@@ -86,6 +86,7 @@ struct CascadeArgs {
   const double *const *Z = nullptr;  // per film layer: nbatch x 2neq_pw impedances
   const double *const *J = nullptr;  // per structured layer: nbatch x (2neq_pw x modes), F-order
   const double *const *Jd = nullptr; // per structured layer: nbatch x (modes x 2neq_pw)
+  const int64_t *rows = nullptr;     // [2 nlayers] J, Jd of a layer row-major per point (null: none)
   const double *heights = nullptr;   // [nbatch * nlayers]: per stack and layer, over the period
   const double *Zair = nullptr;      // nbatch x 2neq_pw: air reference impedances
   const double *d_minus = nullptr;   // nbatch x 2neq_pw incident amplitudes (top)

@@ -243,6 +243,14 @@ int emu_star_cascade_batch(emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_
                            const double *Zair, const double *d_minus, const int64_t *nprop, double *R_net,
                            double *T_net, double *a_list, double *r_list, double *t_list);
 
+/* The same, where row_major[2 l] and row_major[2 l + 1] (NULL: none) say that
+ * layer l's J and J_dagger are row-major per point (C order). */
+int emu_star_cascade_rows(emu_ctx *ctx, int64_t nbatch, int64_t nlayers, int64_t neq_PW, const int64_t *kind,
+                           const int64_t *nmodes, const double *const *kz, const double *const *Z,
+                           const double *const *J, const double *const *J_dagger, const int64_t *row_major, const double *heights,
+                           const double *Zair, const double *d_minus, const int64_t *nprop, double *R_net,
+                           double *T_net, double *a_list, double *r_list, double *t_list);
+
 /* Refractive indices of nq (material, wavelength) queries in one launch
  * (replaces Material.n of backend/materials.py:129-170 evaluated once per
  * wavelength point: linear interpolation of tables with interp1d's segment
