@@ -150,6 +150,39 @@ static void scaled_copy(bool row_major, int nb, int rows, int cols, const zd *X,
   EMU_LAUNCH_CHECK();
 }
 
+// out = M v per point (M r x k column-major): 64 rows per workgroup, its 16
+// waves take every 16th column, eight loads in flight, and add through LDS.  The
+// chain of flux products is one after the other and latency-bound; the 64 x 64
+// tiles of k_zgemm_nn took 8 us for one point of 40 rows and 24 to 26 us for 64
+// points of 98 to 200 rows.
+__global__ __launch_bounds__(1024) void k_matvec(int r, int k, const zd *__restrict__ M, const zd *__restrict__ v,
+                                                 zd *__restrict__ out) {
+  __shared__ zd red[16][64];
+  const int b = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = blockIdx.x * 64 + lane, rc = min(row, r - 1);
+  const zd *Mb = M + (int64_t)b * r * k, *vb = v + (int64_t)b * k;
+  zd acc = zmk(0, 0);
+  for (int c0 = wave; c0 < k; c0 += 128) {
+    zd a[8], x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = min(c0 + 16 * u, k - 1);
+      a[u] = Mb[rc + (int64_t)c * r];
+      x[u] = vb[c];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (c0 + 16 * u < k) acc = zfma(a[u], x[u], acc);
+  }
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && row < r) {
+#pragma unroll
+    for (int w = 1; w < 16; ++w) acc = zadd(acc, red[w][lane]);
+    out[(int64_t)b * r + row] = acc;
+  }
+}
+
 // principal square root with the C99 csqrt conventions (signed zeros)
 __device__ __forceinline__ zd zsqrt(zd z) {
   if (z.x == 0.0 && z.y == 0.0) return zmk(0.0, z.y);
@@ -314,9 +347,9 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
     EMU_HIP(hipMemcpyAsync(p, src, sizeof(zd) * count, hipMemcpyHostToDevice, upl.st ? upl.st : s));
     return p;
   };
-  // 1. interface matrices of every layer against air
+  // 1. interface matrices of a layer against air
   std::vector<Lay> lay(L);
-  for (int i = 0; i < L; ++i) {
+  auto interface = [&](int i) {
     Lay &l = lay[i];
     l.kind = (int)a.kind[i];
     l.dim = l.kind == 0 ? d : (int)a.nmodes[i];
@@ -337,7 +370,7 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
       hipLaunchKernelGGL(k_film_rt, dim3((unsigned)(((int64_t)d * d + 255) / 256), nb), dim3(256), 0, s, d, Zair,
                          Z, l.R12, l.T12, l.R21, l.T21);
       EMU_LAUNCH_CHECK();
-      continue;
+      return;
     }
     // r_t_mat_tf_ns: A = diag(zs) J, B = J^dagger diag(zs), D = I + B A
     zd *J = up(t + "J", a.J[i], (size_t)nb * d * m);
@@ -364,7 +397,11 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
     affine(nb, m, m, Dinv, (int64_t)m * m, nullptr, 0, nullptr, 0, zmk(2, 0), zmk(-1, 0), l.R21, (int64_t)m * m, s);
     launch_gemm_nn(nb, d, m, m, zmk(2, 0), A, d, (int64_t)d * m, Dinv, m, (int64_t)m * m, zero, l.T21, d,
                    (int64_t)d * m, s);
-  }
+    };
+  // Layer by layer from the bottom: its interface matrices, then the net
+  // matrices through it, so that the chain of the layers below fills the wait
+  // for the next layer's upload.
+  interface(0);
   // 2. net matrices bottom-up through the infinitesimal air gaps (stack.py:204-278)
   int tr = d, tc = d;  // tnet shape
   zd *tnet = lay[0].T12;
@@ -410,6 +447,7 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
     it21_list.push_back(it21);
   };
   for (int i = 1; i < L - 1; ++i) {
+    interface(i);
     air_gap(i);
     const Lay &l = lay[i];
     const int m = l.dim;
@@ -443,6 +481,7 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
     rdim.push_back(d);
     it12_list.push_back(it12);
   }
+  interface(L - 1);
   air_gap(L - 1);
   (void)rd;
   // 3. fluxes (stack.py:285-427)
@@ -450,7 +489,8 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
   zd *dflux = c->buf<zd>("cs_down", (size_t)nflux * nb);
   zd *uflux = c->buf<zd>("cs_up", nb);
   auto matvec = [&](const zd *M, int r, int k, const zd *v, zd *out) {
-    launch_gemm_nn(nb, r, 1, k, one, M, r, (int64_t)r * k, v, k, k, zero, out, r, r, s);
+    hipLaunchKernelGGL(k_matvec, dim3((r + 63) / 64, nb), dim3(1024), 0, s, r, k, M, v, out);
+    EMU_LAUNCH_CHECK();
   };
   zd *vplus = c->buf<zd>("cs_vplus", (size_t)nb * d);
   hipLaunchKernelGGL(k_flux, dim3(nb), dim3(256), 0, s, nb, P, dm_, nullptr, (int64_t)d, dnpi, 0, dflux);

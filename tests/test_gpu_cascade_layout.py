@@ -49,3 +49,20 @@ def test_layouts(gpu_ctx, nb, P, m):
                 # the same kernels on the same numbers, but tiles may differ with the batch: rounding
                 # of sums of 33 products through three solves of random (condition ~ 1e3) matrices
                 assert np.abs(x[b] - y[0]).max() <= 1e-9 * max(1.0, np.abs(x[b]).max())
+
+
+@pytest.mark.parametrize('nb,P,m', [(1, 1, 1), (2, 8, 17), (2, 33, 64), (3, 10, 130), (2, 70, 200)])
+def test_flux_products(gpu_ctx, nb, P, m):
+    """r and the last t are those of the nets applied to the incident
+    amplitudes (products of 2 to 200 columns on the device)."""
+    args = _inputs(nb, P, m)
+    a, r, t, R, T = gpu_ctx.star_cascade(*args, want_nets=True)
+    n = args[8][0, 0]
+    prop = np.arange(2 * P) % P < n
+    for b in range(nb):
+        v = args[7][b]
+        down = np.sum(np.abs(v[prop]) ** 2)
+        # one product in another order: 140 roundings of its terms
+        assert abs(r[b] - np.sum(np.abs((R[b] @ v)[prop]) ** 2) / down) <= 1e-12 * max(1, r[b])
+        # three products one after the other against the product of the matrices (condition ~ 1e3)
+        assert abs(t[b, -1] - np.sum(np.abs((T[b] @ v)[prop]) ** 2) / down) <= 1e-9 * max(1, t[b, -1])
