@@ -60,7 +60,7 @@ struct KTime {
 // Gram-Schmidt pass; every `every`-th sweep is recorded.  Classes: 0 forward
 // solve (k_fwd), 1 backward solve (k_bwd), 2 Gram-Schmidt projection
 // (k_atb_mfma16; k_atb_tall for single vectors), 3 Gram-Schmidt update
-// (k_combine; k_sub_vh_blk for single vectors), 4 sparse M product of the
+// (k_combine; k_sub_vh for single vectors), 4 sparse M product of the
 // Krylov block (k_spmm_il; k_spmm for single vectors); per class: dispatches,
 // milliseconds, algorithmic bytes.
 struct Profiler {
@@ -323,21 +323,20 @@ void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64
 void launch_gemm_nn(int nb, int64_t M, int N, int K, zd alpha, const zd *A, int64_t lda, int64_t sA,
                     const zd *B, int64_t ldb, int64_t sB, zd beta, zd *C, int64_t ldc, int64_t sC,
                     hipStream_t s);
-// w[b] -= V[b][:, 0:k] h[b]  (h device, [b][hstride])
-void launch_sub_vh(int nb, int64_t n, int k, const zd *V, int64_t ldv, int64_t sV, const zd *h,
-                   int64_t sh, zd *w, int64_t sw, hipStream_t s);
-// nrm[b] = ||w[b]||; then w[b] *= 1/nrm[b] written to out[b]
-void launch_norm_scale(int nb, int64_t n, const zd *w, int64_t sw, zd *out, int64_t so,
-                       double *nrm, double *scratch, hipStream_t s);
-void launch_axpy_h(int nb, int k, const zd *h1, const zd *h2, int64_t sh, zd *H, int64_t sH,
-                   hipStream_t s);
 void launch_copy(int nb, int64_t n, const zd *src, int64_t ss, zd *dst, int64_t sd, hipStream_t s);
 // exchange two ranges of n elements (two batch slots' data)
 void launch_swap(int64_t n, zd *a, zd *b, hipStream_t s);
 void launch_swap_i32(int64_t n, int32_t *a, int32_t *b, hipStream_t s);
-// block Gram-Schmidt: W[:, :bq] -= V[:, :k] H[:k, :bq]
-void launch_sub_vh_blk(int nb, int64_t n, int k, int bq, const zd *V, int64_t ldv, int64_t sV, const zd *H,
-                       int64_t ldh, int64_t sH, zd *W, int64_t ldw, int64_t sW, hipStream_t s, KTime kt = {});
+// w[b] -= V[b][:, 0:k] h[b]
+void launch_sub_vh(int nb, int64_t n, int k, const zd *V, int64_t ldv, int64_t sV, const zd *h, int64_t sh, zd *w,
+                   int64_t sw, hipStream_t s, KTime kt = {});
+// The whole Gram-Schmidt step of one vector (two passes against V[:, :k], H[:k]
+// and H[k] = |w|, w normalised) for small batches; false if it is not one.
+// h1: k values per instance, npart: (n + 63) / 64 per instance; kp, ks: of the
+// two passes.
+bool launch_cgs1(int nb, int64_t n, int k, const zd *V, int64_t sV, zd *w, int64_t sw, zd *scratch,
+                 size_t scratch_elems, zd *h1, int64_t sh, zd *H, int64_t sH, double *npart, int32_t *bad,
+                 hipStream_t s, const KTime *kp, const KTime *ks);
 // Delayed block Gram-Schmidt (block size bq = 2, 4 or 8).  The projection
 // C[b] (M x N) = A[b]^H B[b], N = bq or 2 bq columns
 void launch_proj(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64_t sA, const zd *B, int64_t ldb,

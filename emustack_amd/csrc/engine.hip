@@ -454,11 +454,6 @@ DevMesh *mesh_load(Ctx *c, const std::string &path, int leaf) {
 }
 
 // ---------------------------------------------------------------- assembly
-__global__ void k_store_norm(int nb, const double *__restrict__ nrm, zd *__restrict__ dst, int64_t sd) {
-  int b = threadIdx.x + blockIdx.x * blockDim.x;
-  if (b < nb) dst[b * sd] = zmk(nrm[b], 0.0);
-}
-
 static void upload_params(Ctx *c, DevMesh &dm, int nb, int ntyp, const double *pp, const double *qq,
                           const double *shift, const double *bloch, zd **dpp, zd **dqq, zd **dsh, double **dbl) {
   *dpp = c->buf<zd>("pp", (size_t)nb * ntyp);
@@ -888,6 +883,7 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
   zd *Hd = c->buf<zd>("ks_H", (size_t)nb * sH);
   zd *H2 = c->buf<zd>("ks_H2", (size_t)nb * ld * bq);
   zd *gpart = c->buf<zd>("ks_gpart", (size_t)nb * bq * bq * gram_blocks(n));
+  double *npart = delayed ? nullptr : c->buf<double>("ks_npart", (size_t)nb * ((n + 63) / 64));
   zd *Ri = c->buf<zd>("ks_Ri", (size_t)nb * bq * bq);
   zd *R1 = c->buf<zd>("ks_R1", (size_t)nb * bq * bq);
   zd *Rf = c->buf<zd>("ks_Rf", (size_t)nb * bq * bq);
@@ -1000,17 +996,23 @@ static EigResult krylov_schur(Ctx *c, DevMesh &dm, int nb, int nev, int m, int b
         res.steps += 1;
         continue;
       }
-      // block CGS, two passes
-      for (int pass = 0; pass < 2; ++pass) {
-        zd *hc = pass == 0 ? Hd + (int64_t)j * ld : H2;
-        int64_t hld = pass == 0 ? ld : ld, hs = pass == 0 ? sH : (int64_t)ld * bq;
-        launch_atb(nact, n, j + bq, bq, V, n, sV, Wn, n, sV, hc, hld, hs, true, atbs, atb_elems, s,
-                   pf ? pf->time(2, nbd * 16.0 * nd * (j + 2 * bq)) : KTime{});
-        launch_sub_vh_blk(nact, n, j + bq, bq, V, n, sV, hc, hld, hs, Wn, n, sV, s,
-                          pf ? pf->time(3, nbd * 16.0 * nd * (j + 3 * bq)) : KTime{});
+      // single vectors: two passes of classical Gram-Schmidt
+      zd *hc = Hd + (int64_t)j * ld;
+      KTime kp[2], ks[2];
+      for (int pass = 0; pf && pass < 2; ++pass) {
+        kp[pass] = pf->time(2, nbd * 16.0 * nd * (j + 2));
+        ks[pass] = pf->time(3, nbd * 16.0 * nd * (j + 3));
       }
-      launch_block_copy(nact, j + bq, bq, H2, ld, (int64_t)ld * bq, Hd + (int64_t)j * ld, ld, sH, true, s);
-      block_cholqr2(nact, n, bq, Wn, sV, gpart, 0, Ri, R1, Rf, bad, s, nullptr, HDest{j, j, nullptr, 0, Hd, ld, sH});
+      if (!launch_cgs1(nact, n, j + 1, V, sV, Wn, sV, atbs, atb_elems, H2, ld, hc, sH, npart, bad, s, kp, ks)) {
+        for (int pass = 0; pass < 2; ++pass) {
+          zd *h = pass == 0 ? hc : H2;
+          const int64_t hs = pass == 0 ? sH : ld;
+          launch_atb(nact, n, j + 1, 1, V, n, sV, Wn, n, sV, h, ld, hs, true, atbs, atb_elems, s, kp[pass]);
+          launch_sub_vh(nact, n, j + 1, V, n, sV, h, hs, Wn, sV, s, ks[pass]);
+        }
+        launch_block_copy(nact, j + 1, 1, H2, ld, ld, hc, ld, sH, true, s);
+        block_cholqr2(nact, n, bq, Wn, sV, gpart, 0, Ri, R1, Rf, bad, s, nullptr, HDest{j, j, nullptr, 0, Hd, ld, sH});
+      }
       res.ops += (int64_t)nact * bq;
       res.steps += 1;
     }

@@ -371,25 +371,19 @@ __global__ __launch_bounds__(256) void k_atb_mfma_wide(int64_t K, int M, int N, 
   }
 }
 
-// ------------------------------------------ C = op(A)^T B for N <= 8 columns
+// ------------------------------------------ C = op(A)^T b for one vector
 // The Gram-Schmidt projection h = V^H w: A (K x M) is the Krylov basis, read
-// once from HBM; B (K x NQ) is the new block.  A workgroup owns 64 columns of
-// A and one K chunk.  Per 32-row step it stages the 32 x 64 tile of A (read
-// along the rows, coalesced) and the 32 x NQ tile of B in LDS; lane c of each
-// wave then accumulates column c against all NQ columns of B over the rows of
-// its wave (rows w, w + 4, ...; the B reads are wave-uniform LDS broadcasts).
-// The next tile is fetched into registers while the current one is used.  At
-// the end the four waves' sums are combined in LDS and written as the chunk's
-// partial product; k_atb_reduce adds the chunks.
-// CPT columns of A per thread: a tile is 64 CPT columns x 32 / CPT rows (the
-// same 2048 elements); with CPT = 2 every B value read from LDS feeds two
-// columns, halving the LDS traffic per FMA for N = 16.
-template <int NQ, int CPT>
+// once from HBM; B is the new vector.  A workgroup owns 64 columns of A and one
+// K chunk.  Per 32-row step it stages the 32 x 64 tile of A (read along the
+// rows, coalesced) and 32 values of B in LDS; lane c of each wave then
+// accumulates column c over the rows of its wave (rows w, w + 4, ...).  The next
+// tile is fetched into registers while the current one is used.  At the end the
+// four waves' sums are combined in LDS and written as the chunk's partial
+// product, added by k_atb_reduce or k_cgs_sub.
 __global__ __launch_bounds__(256) void k_atb_tall(int64_t K, int M, int64_t kchunk, const zd *__restrict__ A,
-                                                  int64_t lda, int64_t sA, const zd *__restrict__ B, int64_t ldb,
-                                                  int64_t sB, int conjA, zd *__restrict__ part) {
-  static_assert(NQ >= 1 && NQ <= 16, "tall kernel covers N <= 16");
-  constexpr int TM = 64 * CPT, TK = 32 / CPT, CG = 256 / TK;  // CG column groups in the staging map
+                                                  int64_t lda, int64_t sA, const zd *__restrict__ B, int64_t sB,
+                                                  int conjA, zd *__restrict__ part) {
+  constexpr int TM = 64, TK = 32;
   const int m0 = blockIdx.x * TM;
   const int chunk = blockIdx.y, nchunk = gridDim.y;
   const int b = blockIdx.z;
@@ -397,10 +391,10 @@ __global__ __launch_bounds__(256) void k_atb_tall(int64_t K, int M, int64_t kchu
   const zd *Ab = A + b * sA;
   const zd *Bb = B + b * sB;
   __shared__ zd As[TK][TM + 1];
-  __shared__ zd Bs[TK][NQ];
+  __shared__ zd Bs[TK];
   const int64_t kb = chunk * kchunk, ke = min(K, kb + kchunk);
-  const int lr = tid % TK, lc = tid / TK;  // staging: row lr, columns lc + CG i
-  zd ra[8], rb[(TK * NQ + 255) / 256];
+  const int lr = tid % TK, lc = tid / TK;  // staging: row lr, columns lc + 8 i
+  zd ra[8], rb;
   // Loads are unconditional from clamped (in-range) addresses, and the
   // out-of-range values are zeroed afterwards: a load inside a branch makes
   // the compiler wait for it before the branch merges, which serialises the
@@ -411,70 +405,32 @@ __global__ __launch_bounds__(256) void k_atb_tall(int64_t K, int M, int64_t kchu
     const int64_t kc = okk ? k : ke - 1;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int m = m0 + lc + CG * i;
+      const int m = m0 + lc + 8 * i;
       const zd v = Ab[kc + (int64_t)min(m, M - 1) * lda];
       ra[i] = (okk && m < M) ? v : zmk(0, 0);
     }
-#pragma unroll
-    for (int i = 0; i < (TK * NQ + 255) / 256; ++i) {
-      const int idx = tid + 256 * i, r = idx % TK, q = idx / TK;
-      const bool ok = q < NQ && k0 + r < ke;
-      const zd v = Bb[(ok ? k0 + r : ke - 1) + (int64_t)min(q, NQ - 1) * ldb];
-      rb[i] = ok ? v : zmk(0, 0);
-    }
+    const zd v = Bb[kc];
+    rb = okk ? v : zmk(0, 0);
   };
-  zd acc[CPT][NQ];
-#pragma unroll
-  for (int c = 0; c < CPT; ++c)
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) acc[c][q] = zmk(0, 0);
+  zd acc = zmk(0, 0);
   if (kb < ke) fetch(kb);
   for (int64_t k0 = kb; k0 < ke; k0 += TK) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) As[lr][lc + CG * i] = conjA ? zconj(ra[i]) : ra[i];
-#pragma unroll
-    for (int i = 0; i < (TK * NQ + 255) / 256; ++i) {
-      const int idx = tid + 256 * i;
-      if (idx < TK * NQ) Bs[idx % TK][idx / TK] = rb[i];
-    }
+    for (int i = 0; i < 8; ++i) As[lr][lc + 8 * i] = conjA ? zconj(ra[i]) : ra[i];
+    if (lc == 0) Bs[lr] = rb;
     __syncthreads();
     if (k0 + TK < ke) fetch(k0 + TK);
 #pragma unroll
-    for (int kk = wv; kk < TK; kk += 4) {
-      zd a[CPT];
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) a[c] = As[kk][lane + 64 * c];
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        const zd bq = Bs[kk][q];
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) acc[c][q] = zfma(a[c], bq, acc[c][q]);
-      }
-    }
+    for (int kk = wv; kk < TK; kk += 4) acc = zfma(As[kk][lane], Bs[kk], acc);
   }
   __syncthreads();
-  // combine the four waves, 64 columns and eight columns of B at a time (LDS
-  // of the A tile reused: 4 x 64 x 8 <= TK x (TM + 1))
   zd *red = &As[0][0];
-  constexpr int QH = NQ < 8 ? NQ : 8;
-#pragma unroll
-  for (int c = 0; c < CPT; ++c)
-#pragma unroll
-    for (int h = 0; h < NQ; h += QH) {
-#pragma unroll
-      for (int q = 0; q < QH; ++q) red[(wv * 64 + lane) * QH + q] = acc[c][h + q];
-      __syncthreads();
-      for (int o = tid; o < 64 * QH; o += 256) {
-        const int cc = o % 64, q = o / 64;
-        zd sum = red[cc * QH + q];
-#pragma unroll
-        for (int w = 1; w < 4; ++w) sum = zadd(sum, red[(w * 64 + cc) * QH + q]);
-        const int m = m0 + 64 * c + cc;
-        if (m < M) part[(((int64_t)b * nchunk + chunk) * NQ + h + q) * M + m] = sum;
-      }
-      __syncthreads();
-    }
+  red[wv * 64 + lane] = acc;
+  __syncthreads();
+  if (wv == 0 && m0 + lane < M)
+    part[((int64_t)b * nchunk + chunk) * M + m0 + lane] =
+        zadd(zadd(zadd(acc, red[64 + lane]), red[128 + lane]), red[192 + lane]);
 }
 
 // Exchange two equal ranges (the data of two batch slots).
@@ -626,6 +582,28 @@ __global__ __launch_bounds__(256) void k_atb_reduce(int M, int N, int nchunk, co
   }
 }
 
+// Partial products A^H b of the K chunks (part[b][chunk][M]), at most `most`
+// chunks; returns their number.
+static int atb_partials(int nb, int64_t K, int M, const zd *A, int64_t lda, int64_t sA, const zd *B, int64_t sB,
+                        bool conjA, int64_t most, zd *scratch, size_t scratch_elems, hipStream_t s,
+                        KTime kt) {
+  const int kstep = 32;
+  const int tiles = (M + 63) / 64;
+  const int64_t per = (int64_t)nb * M;
+  const int64_t maxchunk = std::max<int64_t>(1, (int64_t)(scratch_elems / std::max<int64_t>(per, 1)));
+  const int64_t want = std::max<int64_t>(1, 2048 / std::max(1, tiles * nb));
+  int64_t nchunk = std::min<int64_t>(std::min<int64_t>(want, maxchunk), (K + kstep - 1) / kstep);
+  nchunk = std::max<int64_t>(1, std::min<int64_t>(nchunk, most));
+  int64_t kchunk = (K + nchunk - 1) / nchunk;
+  kchunk = ((kchunk + kstep - 1) / kstep) * kstep;
+  nchunk = (K + kchunk - 1) / kchunk;
+  if ((size_t)(nchunk * per) > scratch_elems) throw HipError("atb: scratch too small");
+  hipExtLaunchKernelGGL(k_atb_tall, dim3((unsigned)tiles, (unsigned)nchunk, nb), dim3(256), 0, s, kt.a, kt.b, 0, K, M,
+                        kchunk, A, lda, sA, B, sB, conjA ? 1 : 0, scratch);
+  EMU_LAUNCH_CHECK();
+  return (int)nchunk;
+}
+
 void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64_t sA, const zd *B,
                 int64_t ldb, int64_t sB, zd *C, int64_t ldc, int64_t sC, bool conjA, zd *scratch,
                 size_t scratch_elems, hipStream_t s, KTime kt) {
@@ -657,24 +635,9 @@ void launch_atb(int nb, int64_t K, int M, int N, const zd *A, int64_t lda, int64
     EMU_LAUNCH_CHECK();
     return;
   }
-  const int kstep = 32;
-  const int tiles = (M + 63) / 64;
-  int64_t per = (int64_t)nb * M * N;
-  int64_t maxchunk = std::max<int64_t>(1, (int64_t)(scratch_elems / std::max<int64_t>(per, 1)));
-  int64_t want = std::max<int64_t>(1, 2048 / std::max(1, tiles * nb));
-  int64_t nchunk = std::min<int64_t>(std::min<int64_t>(want, maxchunk), (K + kstep - 1) / kstep);
-  nchunk = std::max<int64_t>(1, std::min<int64_t>(nchunk, 256));
-  int64_t kchunk = (K + nchunk - 1) / nchunk;
-  kchunk = ((kchunk + kstep - 1) / kstep) * kstep;
-  nchunk = (K + kchunk - 1) / kchunk;
-  if ((size_t)(nchunk * per) > scratch_elems) throw HipError("atb: scratch too small");
-  dim3 g((unsigned)tiles, (unsigned)nchunk, nb), t(256);
-  hipExtLaunchKernelGGL((k_atb_tall<1, 1>), g, t, 0, s, kt.a, kt.b, 0, K, M, kchunk, A, lda, sA, B, ldb, sB,
-                        conjA ? 1 : 0, scratch);
-  EMU_LAUNCH_CHECK();
-  const int64_t tot = (int64_t)M * N;
-  hipLaunchKernelGGL(k_atb_reduce, dim3((unsigned)((tot + 63) / 64), nb), dim3(256), 0, s, M, N, (int)nchunk,
-                     scratch, C, ldc, sC);
+  const int nchunk = atb_partials(nb, K, M, A, lda, sA, B, sB, conjA, 256, scratch, scratch_elems, s, kt);
+  hipLaunchKernelGGL(k_atb_reduce, dim3((unsigned)((M + 63) / 64), nb), dim3(256), 0, s, M, N, nchunk, scratch, C, ldc,
+                     sC);
   EMU_LAUNCH_CHECK();
 }
 
@@ -939,88 +902,6 @@ void launch_gemm_nn(int nb, int64_t M, int N, int K, zd alpha, const zd *A, int6
   EMU_LAUNCH_CHECK();
 }
 
-// ------------------------------------------------------- w -= V[:, :k] h
-__global__ __launch_bounds__(256) void k_sub_vh(int64_t n, int k, const zd *__restrict__ V, int64_t ldv,
-                                                int64_t sV, const zd *__restrict__ h, int64_t sh,
-                                                zd *__restrict__ w, int64_t sw) {
-  __shared__ zd hs[1024];
-  const int b = blockIdx.y;
-  for (int i = threadIdx.x; i < k && i < 1024; i += blockDim.x) hs[i] = h[b * sh + i];
-  __syncthreads();
-  int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const zd *Vb = V + b * sV;
-  zd acc = w[b * sw + r];
-  for (int c = 0; c < k; ++c) acc = zfms(Vb[r + (int64_t)c * ldv], hs[c], acc);
-  w[b * sw + r] = acc;
-}
-
-void launch_sub_vh(int nb, int64_t n, int k, const zd *V, int64_t ldv, int64_t sV, const zd *h, int64_t sh,
-                   zd *w, int64_t sw, hipStream_t s) {
-  if (k > 1024) throw HipError("sub_vh: Krylov dimension above 1024");
-  dim3 g((unsigned)((n + 255) / 256), nb);
-  hipLaunchKernelGGL(k_sub_vh, g, dim3(256), 0, s, n, k, V, ldv, sV, h, sh, w, sw);
-  EMU_LAUNCH_CHECK();
-}
-
-// -------------------------------------------------- norm and normalisation
-__global__ __launch_bounds__(256) void k_norm_partial(int64_t n, const zd *__restrict__ w, int64_t sw,
-                                                      double *__restrict__ part) {
-  __shared__ double red[256];
-  const int b = blockIdx.y;
-  double acc = 0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    zd v = w[b * sw + i];
-    acc += v.x * v.x + v.y * v.y;
-  }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[b * gridDim.x + blockIdx.x] = red[0];
-}
-
-__global__ __launch_bounds__(256) void k_norm_scale(int64_t n, int nparts, const double *__restrict__ part,
-                                                    const zd *__restrict__ w, int64_t sw, zd *__restrict__ out,
-                                                    int64_t so, double *__restrict__ nrm) {
-  __shared__ double tot;
-  const int b = blockIdx.y;
-  if (threadIdx.x == 0) {
-    double acc = 0;
-    for (int i = 0; i < nparts; ++i) acc += part[b * nparts + i];
-    tot = sqrt(acc);
-    if (blockIdx.x == 0) nrm[b] = tot;
-  }
-  __syncthreads();
-  const double inv = tot > 0 ? 1.0 / tot : 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    out[b * so + i] = zscale(w[b * sw + i], inv);
-}
-
-void launch_norm_scale(int nb, int64_t n, const zd *w, int64_t sw, zd *out, int64_t so, double *nrm,
-                       double *scratch, hipStream_t s) {
-  const int nparts = 64;
-  hipLaunchKernelGGL(k_norm_partial, dim3(nparts, nb), dim3(256), 0, s, n, w, sw, scratch);
-  EMU_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_norm_scale, dim3(nparts, nb), dim3(256), 0, s, n, nparts, scratch, w, sw, out, so, nrm);
-  EMU_LAUNCH_CHECK();
-}
-
-// H[b][0:k] = h1 + h2
-__global__ void k_axpy_h(int k, const zd *__restrict__ h1, const zd *__restrict__ h2, int64_t sh,
-                         zd *__restrict__ H, int64_t sH) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int b = blockIdx.y;
-  if (i < k) H[b * sH + i] = zadd(h1[b * sh + i], h2[b * sh + i]);
-}
-
-void launch_axpy_h(int nb, int k, const zd *h1, const zd *h2, int64_t sh, zd *H, int64_t sH, hipStream_t s) {
-  hipLaunchKernelGGL(k_axpy_h, dim3((k + 255) / 256, nb), dim3(256), 0, s, k, h1, h2, sh, H, sH);
-  EMU_LAUNCH_CHECK();
-}
-
 __global__ void k_copy(int64_t n, const zd *__restrict__ src, int64_t ss, zd *__restrict__ dst, int64_t sd) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   int b = blockIdx.y;
@@ -1038,52 +919,143 @@ void launch_copy(int nb, int64_t n, const zd *src, int64_t ss, zd *dst, int64_t 
 namespace emu {
 
 // ---------------------------------------------- block Gram-Schmidt helpers
-// W[b][:, q] -= sum_{c<k} V[b][:, c] H[b][c, q],  q < bq  (thread per row,
-// H staged through LDS in chunks of 64 rows)
-template <int BQ>
-__global__ __launch_bounds__(256) void k_sub_vh_blk(int64_t n, int k, const zd *__restrict__ V, int64_t ldv,
-                                                    int64_t sV, const zd *__restrict__ H, int64_t ldh, int64_t sH,
-                                                    zd *__restrict__ W, int64_t ldw, int64_t sW) {
-  __shared__ zd hs[64][BQ];
+// w[b] -= sum_{c<k} V[b][:, c] h[b][c]  (thread per row, h staged through LDS 64 values at a time)
+__global__ __launch_bounds__(256) void k_sub_vh(int64_t n, int k, const zd *__restrict__ V, int64_t ldv, int64_t sV,
+                                                const zd *__restrict__ h, int64_t sh, zd *__restrict__ w,
+                                                int64_t sw) {
+  __shared__ zd hs[64];
   const int b = blockIdx.y;
   const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const zd *Vb = V + b * sV;
-  const zd *Hb = H + b * sH;
-  zd acc[BQ];
-#pragma unroll
-  for (int q = 0; q < BQ; ++q) acc[q] = (r < n) ? W[b * sW + q * ldw + r] : zmk(0, 0);
+  zd acc = r < n ? w[b * sw + r] : zmk(0, 0);
   for (int c0 = 0; c0 < k; c0 += 64) {
     const int cn = min(64, k - c0);
     __syncthreads();
-    for (int idx = threadIdx.x; idx < 64 * BQ; idx += blockDim.x) {
-      int c = idx / BQ, q = idx - c * BQ;
-      hs[c][q] = c < cn ? Hb[(c0 + c) + (int64_t)q * ldh] : zmk(0, 0);
-    }
+    if (threadIdx.x < 64) hs[threadIdx.x] = (int)threadIdx.x < cn ? h[b * sh + c0 + threadIdx.x] : zmk(0, 0);
     __syncthreads();
     if (r < n)
-      for (int c = 0; c < cn; ++c) {
-        const zd v = Vb[r + (int64_t)(c0 + c) * ldv];
-#pragma unroll
-        for (int q = 0; q < BQ; ++q) acc[q] = zfms(v, hs[c][q], acc[q]);
-      }
+      for (int c = 0; c < cn; ++c) acc = zfms(Vb[r + (int64_t)(c0 + c) * ldv], hs[c], acc);
   }
-  if (r < n)
-#pragma unroll
-    for (int q = 0; q < BQ; ++q) W[b * sW + q * ldw + r] = acc[q];
+  if (r < n) w[b * sw + r] = acc;
 }
 
-void launch_sub_vh_blk(int nb, int64_t n, int k, int bq, const zd *V, int64_t ldv, int64_t sV, const zd *H,
-                       int64_t ldh, int64_t sH, zd *W, int64_t ldw, int64_t sW, hipStream_t s, KTime kt) {
-  dim3 g((unsigned)((n + 255) / 256), nb);
-  dim3 t(256);
-  switch (bq) {
-    case 1: hipExtLaunchKernelGGL(k_sub_vh_blk<1>, g, t, 0, s, kt.a, kt.b, 0, n, k, V, ldv, sV, H, ldh, sH, W, ldw, sW); break;
-    case 2: hipExtLaunchKernelGGL(k_sub_vh_blk<2>, g, t, 0, s, kt.a, kt.b, 0, n, k, V, ldv, sV, H, ldh, sH, W, ldw, sW); break;
-    case 4: hipExtLaunchKernelGGL(k_sub_vh_blk<4>, g, t, 0, s, kt.a, kt.b, 0, n, k, V, ldv, sV, H, ldh, sH, W, ldw, sW); break;
-    case 8: hipExtLaunchKernelGGL(k_sub_vh_blk<8>, g, t, 0, s, kt.a, kt.b, 0, n, k, V, ldv, sV, H, ldh, sH, W, ldw, sW); break;
-    default: throw HipError("sub_vh_blk: block size must be 1, 2, 4 or 8");
-  }
+void launch_sub_vh(int nb, int64_t n, int k, const zd *V, int64_t ldv, int64_t sV, const zd *h, int64_t sh, zd *w,
+                   int64_t sw, hipStream_t s, KTime kt) {
+  hipExtLaunchKernelGGL(k_sub_vh, dim3((unsigned)((n + 255) / 256), nb), dim3(256), 0, s, kt.a, kt.b, 0, n, k, V, ldv,
+                        sV, h, sh, w, sw);
   EMU_LAUNCH_CHECK();
+}
+
+// Two-pass Gram-Schmidt of one vector against k columns on small batches, in
+// five dependent launches instead of ten: the projection's partial sums
+// (k_atb_tall), then k_cgs_sub, in which every workgroup adds them up for
+// itself (k x nchunk values from L2) and subtracts, once more of both, and
+// k_cgs_norm.  A launch in this chain takes 2 to 6 us however little it does
+// (a step of two instances of 1,990 unknowns 92 -> 76 us, of 32 166 -> 157 us).
+// A workgroup has 64 rows; its four waves take every fourth column and add
+// through LDS.  h1: the first pass's coefficients.  LAST: the second pass
+// stores the sum of both to H and its rows' part of |w|^2 to npart.
+template <bool LAST>
+__global__ __launch_bounds__(256) void k_cgs_sub(int n, int k, const zd *__restrict__ V, int64_t sV,
+                                                 const zd *__restrict__ part, int nchunk, zd *__restrict__ h1,
+                                                 int64_t sh, zd *__restrict__ H, int64_t sH, zd *__restrict__ w,
+                                                 int64_t sw, double *__restrict__ npart) {
+  __shared__ zd hs[256], red[3][64];
+  const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, g = tid >> 6;
+  const int row = blockIdx.x * 64 + lane, rc = min(row, n - 1);
+  const zd *Vb = V + b * sV + rc, *pb = part + (int64_t)b * nchunk * k;
+  const zd w0 = w[b * sw + rc];
+  zd acc = zmk(0, 0);
+  for (int c0 = 0; c0 < k; c0 += 256) {
+    const int cn = min(256, k - c0), e = c0 + min(tid, cn - 1);
+    zd h = zmk(0, 0);
+    for (int q = 0; q < nchunk; q += 8) {
+      zd v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = pb[(int64_t)min(q + u, nchunk - 1) * k + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (q + u < nchunk) h = zadd(h, v[u]);
+    }
+    __syncthreads();
+    hs[tid] = tid < cn ? h : zmk(0, 0);
+    if (blockIdx.x == 0 && tid < cn) {
+      if (LAST) H[b * sH + e] = zadd(h1[b * sh + e], h);
+      else h1[b * sh + e] = h;
+    }
+    __syncthreads();
+    for (int c = g; c < cn; c += 32) {
+      zd v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = Vb[(int64_t)(c0 + min(c + 4 * u, cn - 1)) * n];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (c + 4 * u < cn) acc = zfma(v[u], hs[c + 4 * u], acc);
+    }
+  }
+  if (g > 0) red[g - 1][lane] = acc;
+  __syncthreads();
+  if (g > 0) return;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) acc = zadd(acc, red[q][lane]);
+  const zd x = zsub(w0, acc);
+  if (row < n) w[b * sw + row] = x;
+  if (LAST) {
+    double d = row < n ? x.x * x.x + x.y * x.y : 0.0;
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) d += __shfl_xor(d, m, 64);
+    if (lane == 0) npart[(int64_t)b * gridDim.x + blockIdx.x] = d;
+  }
+}
+
+// w /= |w| from the sums of k_cgs_sub; |w| to *hn (a length of zero is replaced
+// by a tiny one and counted, as in k_cholqr)
+__global__ __launch_bounds__(256) void k_cgs_norm(int n, int nparts, const double *__restrict__ npart,
+                                                  zd *__restrict__ w, int64_t sw, zd *__restrict__ hn, int64_t sH,
+                                                  int32_t *__restrict__ bad) {
+  __shared__ double red[4];
+  const int b = blockIdx.y, tid = threadIdx.x;
+  double d = 0;
+  for (int i = tid; i < nparts; i += 256) d += npart[(int64_t)b * nparts + i];
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) d += __shfl_xor(d, m, 64);
+  if ((tid & 63) == 0) red[tid >> 6] = d;
+  __syncthreads();
+  d = (red[0] + red[1]) + (red[2] + red[3]);
+  const bool zero = !(d > 0.0);
+  if (zero) d = 1e-300;
+  const double r = sqrt(d), inv = 1.0 / r;
+  const int row = blockIdx.x * 256 + tid;
+  if (row < n) w[b * sw + row] = zscale(w[b * sw + row], inv);
+  if (blockIdx.x == 0 && tid == 0) {
+    hn[b * sH] = zmk(r, 0.0);
+    if (zero) bad[b] += 1;
+  }
+}
+
+// Where the vectors' 64-row pieces are at most 1,280 workgroups (a fuller chip
+// is bound by the basis' bytes, and the partial sums read again by every
+// workgroup only add to them).  False: not for this size, nothing done.
+bool launch_cgs1(int nb, int64_t n, int k, const zd *V, int64_t sV, zd *w, int64_t sw, zd *scratch,
+                 size_t scratch_elems, zd *h1, int64_t sh, zd *H, int64_t sH, double *npart, int32_t *bad,
+                 hipStream_t s, const KTime *kp, const KTime *ks) {
+  const int64_t blocks = (n + 63) / 64;
+  if (blocks * nb > 1280 || n > INT32_MAX - 256) return false;
+  for (int pass = 0; pass < 2; ++pass) {
+    const int nchunk = atb_partials(nb, n, k, V, n, sV, w, sw, true, 32, scratch, scratch_elems, s, kp[pass]);
+    const KTime kt = ks[pass];
+    if (pass == 0)
+      hipExtLaunchKernelGGL(k_cgs_sub<false>, dim3((unsigned)blocks, nb), dim3(256), 0, s, kt.a, kt.b, 0, (int)n, k, V,
+                            sV, scratch, nchunk, h1, sh, H, sH, w, sw, npart);
+    else
+      hipExtLaunchKernelGGL(k_cgs_sub<true>, dim3((unsigned)blocks, nb), dim3(256), 0, s, kt.a, kt.b, 0, (int)n, k, V,
+                            sV, scratch, nchunk, h1, sh, H, sH, w, sw, npart);
+    EMU_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(k_cgs_norm, dim3((unsigned)((n + 255) / 256), nb), dim3(256), 0, s, (int)n, (int)blocks, npart, w,
+                     sw, H + k, sH, bad);
+  EMU_LAUNCH_CHECK();
+  return true;
 }
 
 // ------------------------------- delayed block Gram-Schmidt (one pass per block)

@@ -287,7 +287,7 @@ int emu_film_modes_batch(emu_ctx *ctx, int64_t nbatch, int64_t npw, const double
  * those launches.  Classes: 0 forward-solve level sweep (k_fwd), 1 backward
  * level sweep (k_bwd), 2 Gram-Schmidt projections (k_atb_mfma16 for
  * blocks of columns, k_atb_tall for single vectors), 3 Gram-Schmidt updates
- * (k_combine; k_sub_vh_blk for single vectors), 4 mass-matrix
+ * (k_combine; k_sub_vh or k_cgs_sub for single vectors), 4 mass-matrix
  * product of the Krylov block (k_spmm_il; k_spmm for single vectors),
  * 5..7 reserved. */
 int emu_profile(emu_ctx *ctx, int enable, int every, double *out);
