@@ -137,6 +137,14 @@ struct SolveTasks {
   int32_t nslot = 0, span = 0;
 };
 
+// The levels at the top of the tree that k_top solves in one launch: offsets
+// and counts of their forward and backward tile tasks, from the lowest up.
+struct TopLevels {
+  static constexpr int kMax = 16;
+  int32_t n = 0;
+  int32_t off[2][kMax] = {}, cnt[2][kMax] = {};  // [0] forward, [1] backward; offsets in records
+};
+
 // Kernel task lists of one factorisation / solve level.
 struct StepPlan {
   int32_t k0;
@@ -206,6 +214,7 @@ struct DevMesh {
   DBuf<InvTile> inv_tiles;           // its products, in dependent phases (first tile, count)
   std::vector<std::pair<int64_t, int64_t>> inv_phases;
   int64_t wsz = 0;                   // entries of their intermediate products per instance
+  TopLevels top;
   std::vector<LevelSched> sched;     // sched[0] = deepest level
   int32_t max_f = 0, max_s = 0;
   // geometry for the plane-wave integrals

@@ -313,6 +313,36 @@ void devmesh_build(DevMesh &dm, hipStream_t s) {
     }
     dm.sched.push_back(L);
   }
+  // The top levels whose fronts have at most 64 pivots (a wave gathers a
+  // front's input in one go) and, together, at most 32 tiles (two per wave; a
+  // level of more has enough workgroups for a launch of its own): all of a
+  // grating's separators, none of a large 2D mesh's.
+  for (size_t l = 0; l < sy.levels.size() && dm.top.n < TopLevels::kMax; ++l) {  // from the root
+    int64_t tiles = 0;
+    bool fits = true;
+    for (int32_t t : sy.levels[l].fronts) {
+      fits = fits && sy.fronts[t].s >= 1 && sy.fronts[t].s <= 64;
+      tiles += (sy.fronts[t].f + 63) / 64;
+    }
+    if (!fits || tiles > 32) break;
+    ++dm.top.n;
+  }
+  if (dm.top.n < 2) dm.top.n = 0;
+  for (int32_t i = 0; i < dm.top.n; ++i)
+    for (int dir = 0; dir < 2; ++dir) {
+      while (tasks.size() % 16) tasks.push_back(-1);
+      dm.top.off[dir][i] = (int32_t)(tasks.size() / 16);
+      for (int32_t t : sy.levels[dm.top.n - 1 - i].fronts) {
+        const FrontInfo &F = sy.fronts[t];
+        for (int32_t r0 = 0; r0 < (dir ? F.s : F.f); r0 += 64) {
+          const SolveTask T{t, r0, 1, -1, -1, F.s, F.f, F.b, io[t], F.pivoff, fv[t], F.uoff};
+          int32_t w[16];
+          std::memcpy(w, &T, sizeof(T));
+          tasks.insert(tasks.end(), w, w + 16);
+        }
+      }
+      dm.top.cnt[dir][i] = (int32_t)(tasks.size() / 16) - dm.top.off[dir][i];
+    }
   // inverted-factor form: offsets, child update-vector map, task lists
   {
     const int64_t accf = nf ? fv[nf - 1] + sy.fronts[nf - 1].f : 0;

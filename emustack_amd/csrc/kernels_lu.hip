@@ -1426,6 +1426,77 @@ static void launch_bwd(const SolveTasks &T, DevMesh &dm, FrontArrays A, int nb, 
                        sy.n, part, (int)T.nslot, x, sx);
 }
 
+// The top levels of a tree of small fronts (a grating's separators), forward to
+// the root and back down, in one launch: a workgroup of 16 waves per instance
+// and right-hand side, a wave per 64-row tile, a barrier per level.  These
+// launches took 3.2 to 4.2 us each however few tiles they had (a grating of
+// 1,990 unknowns at one wavelength 17.9 -> 15.5 ms, at 16 43.0 -> 40.5 ms).  y, x and w are
+// written by some waves and read by others after the barrier, so none of their
+// pointers is restrict or read-only here.
+template <typename FT>
+__global__ __launch_bounds__(1024) void k_top(const SolveTask *__restrict__ tasks, TopLevels L,
+                                              const int32_t *__restrict__ cmap, const int32_t *__restrict__ uidx,
+                                              const FT *__restrict__ inv, int64_t isz, const int4 *__restrict__ gx,
+                                              int64_t npiv, int nrhs, int64_t n, int64_t nw, const zd *__restrict__ bv,
+                                              zd *y, zd *w, zd *x, int64_t sx) {
+  constexpr uint32_t EB = FactorLd<FT>::kBytes;
+  constexpr int NB8 = 8;  // factor columns in flight
+  const int b = blockIdx.x, q = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const zd *bq = bv + ((int64_t)b * nrhs + q) * n;
+  zd *yq = y + ((int64_t)b * nrhs + q) * n, *wq = w + ((int64_t)b * nrhs + q) * nw;
+  zd *xq = x + (int64_t)b * sx + (int64_t)q * n;
+  // acc += F[:, c0 + k] v_k for k = 0..cnt-1, v_k in lane k
+  auto columns = [&](__amdgpu_buffer_rsrc_t F, uint32_t rowb, int ld, int c0, int cnt, zd v, zd acc) {
+    for (int k = 0; k < cnt; k += NB8) {
+      zd a[NB8];
+#pragma unroll
+      for (int u = 0; u < NB8; ++u) a[u] = FactorLd<FT>::ld(F, rowb, (uint32_t)((c0 + min(k + u, cnt - 1)) * ld) * EB);
+#pragma unroll
+      for (int u = 0; u < NB8; ++u)
+        if (k + u < cnt) acc = zfma(a[u], zmk(__shfl(v.x, k + u, 64), __shfl(v.y, k + u, 64)), acc);
+    }
+    return acc;
+  };
+  for (int l = 0; l < L.n; ++l) {
+    for (int t = wave; t < L.cnt[0][l]; t += 16) {
+      const SolveTask T = tasks[L.off[0][l] + t];
+      const int s = T.s, f = T.f, row = T.r0 + lane, rowc = min(row, f - 1);
+      const __amdgpu_buffer_rsrc_t F = buf_view(inv + b * isz + T.ioff, (uint32_t)f * (uint32_t)s * EB);
+      const int2 cr = reinterpret_cast<const int2 *>(cmap)[T.fvoff + rowc];
+      const int4 g = gx[b * npiv + T.pivoff + min(lane, s - 1)];
+      zd v = bq[g.x];
+      if (g.y >= 0) v = zadd(v, wq[g.y]);
+      if (g.z >= 0) v = zadd(v, wq[g.z]);
+      zd acc = columns(F, (uint32_t)rowc * EB, f, 0, s, v, zmk(0, 0));
+      if (row < s) {
+        yq[T.fb + row] = acc;
+      } else if (row < f) {
+        if (cr.x >= 0) acc = zadd(acc, wq[cr.x]);
+        if (cr.y >= 0) acc = zadd(acc, wq[cr.y]);
+        wq[T.uoff + (row - s)] = acc;
+      }
+    }
+    __syncthreads();
+  }
+  for (int l = L.n - 1; l >= 0; --l) {
+    for (int t = wave; t < L.cnt[1][l]; t += 16) {
+      const SolveTask T = tasks[L.off[1][l] + t];
+      const int s = T.s, f = T.f, row = T.r0 + lane;
+      const __amdgpu_buffer_rsrc_t F =
+          buf_view(inv + b * isz + T.ioff + (int64_t)f * s, (uint32_t)f * (uint32_t)s * EB);
+      zd acc = zmk(0, 0);
+      for (int kc = T.r0; kc < f; kc += 64) {
+        const int k = min(kc + lane, f - 1);
+        const zd v = k < s ? yq[T.fb + k] : xq[uidx[T.uoff + k - s]];
+        acc = columns(F, (uint32_t)min(row, s - 1) * EB, s, kc, min(64, f - kc), v, acc);
+      }
+      if (row < s) xq[T.fb + row] = acc;
+    }
+    __syncthreads();
+  }
+}
+
 int64_t solve_ws(const DevMesh &dm) { return std::max<int64_t>(dm.host.sym.nw, 1) + dm.part_rhs; }
 
 // The split task lists for the Krylov solves (one block of at most 8
@@ -1444,7 +1515,11 @@ static void lu_solve_t(DevMesh &dm, int nb, int nrhs, const FT *inv, const int32
   const double fscale = FactorLd<FT>::kBytes / 16.0;  // factor bytes per entry relative to complex128
   // partial sums of split tasks live behind the update vectors in w
   zd *part = w + (int64_t)nb * nrhs * std::max<int64_t>(dm.host.sym.nw, 1);
-  for (const LevelSched &L : dm.sched) {
+  // the dense solves' many right-hand sides fill the launches by themselves,
+  // and a profile times the levels one by one
+  const size_t ntop = prof || nrhs > 8 ? 0 : dm.top.n, nlow = dm.sched.size() - ntop;
+  for (size_t l = 0; l < nlow; ++l) {
+    const LevelSched &L = dm.sched[l];
     const SolveTasks &T = pick_tasks(L.fwd, nrhs);
     const int rc = pick_rc(nrhs, T.cnt, nb);
     KTime kt = prof ? prof->time(0, L.fwd_mat * fscale * nb + L.fwd_vec * vecs) : KTime{};
@@ -1456,7 +1531,13 @@ static void lu_solve_t(DevMesh &dm, int nb, int nrhs, const FT *inv, const int32
     }
   }
   EMU_LAUNCH_CHECK();
-  for (auto it = dm.sched.rbegin(); it != dm.sched.rend(); ++it) {
+  if (ntop > 0) {
+    hipLaunchKernelGGL(k_top<FT>, dim3(nb, nrhs), dim3(1024), 0, s, reinterpret_cast<const SolveTask *>(dm.tasks.p),
+                       dm.top, dm.cmap.p, dm.uidx.p, inv, dm.isz, reinterpret_cast<const int4 *>(gx), dm.host.sym.npiv,
+                       nrhs, dm.host.sym.n, std::max<int64_t>(dm.host.sym.nw, 1), bnew, y, w, x, sx);
+    EMU_LAUNCH_CHECK();
+  }
+  for (auto it = dm.sched.rbegin() + ntop; it != dm.sched.rend(); ++it) {
     const SolveTasks &T = pick_tasks(it->bwd, nrhs);
     const int rc = pick_rc(nrhs, T.cnt, nb);
     KTime kt = prof ? prof->time(1, it->bwd_mat * fscale * nb + it->bwd_vec * vecs) : KTime{};
