@@ -330,13 +330,14 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
   // before them, on a stream of their own; each layer waits for its two (three
   // layers of 98 x 200, 64 points, 120 MB in all: the call 20.7 -> 17.6 ms).
   struct Uploads {
-    hipStream_t st = nullptr;
+    hipStream_t main, st = nullptr;
     hipEvent_t ev = nullptr;
-    ~Uploads() {  // nothing reads the caller's arrays after the call, thrown out of or not
+    ~Uploads() {  // nothing reads the caller's arrays (or `small`) after the call, thrown out of or not
+      (void)hipStreamSynchronize(main);
       if (st) (void)hipStreamSynchronize(st);
       if (ev) (void)hipEventDestroy(ev);
     }
-  } upl;
+  } upl{s};
   if (jmax >= (1u << 20)) {
     if (!c->upload) EMU_HIP(hipStreamCreateWithFlags(&c->upload, hipStreamNonBlocking));
     EMU_HIP(hipEventCreateWithFlags(&upl.ev, hipEventDisableTiming));
