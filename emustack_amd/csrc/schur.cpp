@@ -65,19 +65,26 @@ inline void rotation(cplx a, cplx b, double &c, cplx &s, cplx &r) {
     r = a * (h2 * q);
     return;
   }
-  const double ar = std::hypot(a.real(), a.imag()), br = std::hypot(b.real(), b.imag());
-  if (br == 0) {
+  // far from 1 in size: each phase from its number scaled by a power of two (the
+  // smallest numbers have no digits left for a quotient of modulus one)
+  const double ma = std::max(std::fabs(a.real()), std::fabs(a.imag()));
+  const double mb = std::max(std::fabs(b.real()), std::fabs(b.imag()));
+  if (!(mb > 0)) {
     c = 1;
     s = 0;
     r = a;
     return;
   }
-  const double n = std::hypot(ar, br);
-  const cplx pa = ar > 0 ? cplx(a.real() / ar, a.imag() / ar) : cplx(1);
-  const cplx pb(b.real() / br, -b.imag() / br);
+  const int ea = ma > 0 ? std::ilogb(ma) : 0, eb = std::ilogb(mb), e0 = ma > 0 ? std::max(ea, eb) : eb;
+  const cplx sa(std::ldexp(a.real(), -ea), std::ldexp(a.imag(), -ea));
+  const cplx sb(std::ldexp(b.real(), -eb), std::ldexp(b.imag(), -eb));
+  const double ha = std::hypot(sa.real(), sa.imag()), hb = std::hypot(sb.real(), sb.imag());
+  const cplx pa = ma > 0 ? cplx(sa.real() / ha, sa.imag() / ha) : cplx(1);
+  const cplx pb(sb.real() / hb, -sb.imag() / hb);
+  const double ar = ma > 0 ? std::ldexp(ha, ea - e0) : 0.0, br = std::ldexp(hb, eb - e0), n = std::hypot(ar, br);
   c = ar / n;
   s = mul(pa, pb) * (br / n);
-  r = pa * n;
+  r = pa * std::ldexp(n, e0);
 }
 
 // columns x, y (m complex values): [x y] <- [x y] [c, -s; conj(s), c]
@@ -397,8 +404,13 @@ bool qr(int n, const Mat &h, const Mat &z, int nz, std::vector<Work> &work, int 
 
 // Householder vector of x[0..n-1]: (I - tau w w^H) x = beta e1, w[0] = 1
 void reflector(int n, const cplx *x, cplx *w, double &tau, cplx &beta) {
+  double top = 0;
+  for (int i = 0; i < n; ++i) top = std::max(top, std::max(std::fabs(x[i].real()), std::fabs(x[i].imag())));
+  // numbers whose squares lose digits are scaled by a power of two
+  const int e = top > 0 && (top < 1e-130 || top > 1e130) ? std::ilogb(top) : 0;
+  auto at = [&](int i) { return e ? cplx(std::ldexp(x[i].real(), -e), std::ldexp(x[i].imag(), -e)) : x[i]; };
   double nr = 0;
-  for (int i = 1; i < n; ++i) nr += std::norm(x[i]);
+  for (int i = 1; i < n; ++i) nr += std::norm(at(i));
   w[0] = 1;
   if (nr == 0) {
     tau = 0;
@@ -406,11 +418,13 @@ void reflector(int n, const cplx *x, cplx *w, double &tau, cplx &beta) {
     for (int i = 1; i < n; ++i) w[i] = 0;
     return;
   }
-  const double a0 = std::abs(x[0]), nm = std::sqrt(nr + a0 * a0);
-  const cplx ph = a0 > 0 ? x[0] / a0 : cplx(1);
+  const cplx x0 = at(0);
+  const double a0 = std::abs(x0), nm = std::sqrt(nr + a0 * a0);
+  const cplx ph = a0 > 1e-280 ? x0 / a0 : cplx(1);  // smaller ones have no digits for a phase
   beta = -ph * nm;
-  const cplx u0 = x[0] - beta;  // |u0| = a0 + nm: no cancellation
-  for (int i = 1; i < n; ++i) w[i] = x[i] / u0;
+  const cplx u0 = x0 - beta;  // |u0| = a0 + nm: no cancellation
+  for (int i = 1; i < n; ++i) w[i] = at(i) / u0;
+  if (e) beta = cplx(std::ldexp(beta.real(), e), std::ldexp(beta.imag(), e));
   tau = (a0 + nm) / nm;  // 2 |u0|^2 / ||u||^2
 }
 

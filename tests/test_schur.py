@@ -42,6 +42,10 @@ def _matrix(kind, n):
         a[:k, :k] = g[:k, :k]
         a[2 * k:, 2 * k:] = np.triu(g[2 * k:, 2 * k:], 1) + np.eye(n - 2 * k)
         return a
+    if kind == 'ones':  # rank one: the reduction leaves entries down to the smallest numbers
+        return np.ones((n, n))
+    if kind == 'steep':  # columns of 1e-160 and less on the way
+        return g * 10.0 ** -np.linspace(0, 300, n)[:, None]
     if kind == 'huge':
         return g * 1e150
     return g * 1e-120  # tiny
@@ -49,7 +53,8 @@ def _matrix(kind, n):
 
 @pytest.mark.parametrize('kind,n', [(k, n) for k in ('dense', 'krylov', 'split')
                                     for n in (1, 2, 3, 9, 25, 26, 27, 28, 33, 65, 79, 80, 104, 159, 161, 191, 193,
-                                              319, 321, 504)] + [('huge', 40), ('tiny', 40)])
+                                              319, 321, 504)] + [('huge', 40), ('tiny', 40), ('steep', 40), ('steep', 90), ('ones', 30), ('ones', 90), ('ones', 193),
+                                                                         ('ones', 300)])
 def test_schur_form(kind, n):
     a = _matrix(kind, n)
     rng = np.random.default_rng(n + 1)
