@@ -215,7 +215,11 @@ __device__ __forceinline__ zd zrecip(zd d) {
 //  * every thread forms the reciprocal of its own candidate while the search
 //    runs, each wave reduces its candidates with DPP moves and its winner posts
 //    its row and reciprocal to the wave's LDS slot; one barrier (none when
-//    NW = 1), then every thread picks the winner among the NW slots;
+//    NW = 1), then every thread picks the winner among the NW slots.  There are
+//    two sets of slots, by the parity of the column in its chunk: a wave that
+//    is a step ahead posts to the set that no other wave still reads, and it
+//    cannot be two ahead, as that takes the next step's barrier (a chunk ends
+//    with barriers of its own);
 //  * half a chunk's columns at a time are a ring: a step uses entry 0, writes
 //    the updated entry c to c - 1 and the multiplier (or the finished U entry)
 //    to the last place, so that register indices are compile-time without
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(64 * NW) void k_panel_reg(const int32_t *__restrict
           }
           continue;
         }
-        const int k = k0 + c0 + j0 + jj, pb = jj & 1;
+        const int k = k0 + c0 + j0 + jj, pb = (j0 + jj) & 1;
         // this wave's largest candidate; NaN counts as the smallest value of a
         // row, absent and finished rows below it
         double best = -2.0, a[RPT];

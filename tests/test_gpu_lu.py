@@ -67,6 +67,14 @@ def test_fronts_of_a_cell(gpu_ctx, tmp_path, ntri, leaf):
            tol=1e-11 if leaf == 100000 else 1e-8)
 
 
+@pytest.mark.parametrize('nel', [257, 513])
+def test_dense_front_beyond_two_and_four_thousand_rows(gpu_ctx, nel):
+    """2,056 unknowns: just into the panels of 2,049 to 4,096 candidates.  4,104:
+    the first panel step in memory, the second takes over in registers (n eps
+    times 10 = 9e-12)."""
+    _check(gpu_ctx, _grating(gpu_ctx, nel, 100000), nel, nb=1)
+
+
 def test_zero_pivot_is_replaced_and_counted(gpu_ctx):
     """An all-zero matrix: every pivot is replaced and counted, nothing hangs."""
     mh = _grating(gpu_ctx, 9, 100000)
