@@ -700,7 +700,8 @@ bool qr(int n, const Mat &h, const Mat &z, int nz, std::vector<Work> &work, int 
 static void reorder(int n, const Mat &t, const Mat &z, int nz, const int *sel) {
   alignas(64) double buf[16 * (kPath + 1)];
   std::vector<Path> paths(kPath / 2);
-  std::vector<char> mark(sel, sel + n);
+  std::vector<char> mark(n);
+  for (int i = 0; i < n; ++i) mark[i] = sel[i] != 0;
   for (int top = 0; top < n; ++top) {
     if (mark[top]) continue;
     // the next selected rows, at most half a window of them; they travel together

@@ -77,3 +77,13 @@ def test_schur_form(kind, n):
         near = np.abs(ref[:, None] - np.diag(t)[None, :])
         # a random dense matrix: condition numbers of its eigenvalues up to a few n
         assert near.min(axis=1).max() <= 10 * n * tol * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize('value', [256, -65536, 1 << 30])
+def test_any_nonzero_selects(value):
+    """A row is selected by any value but zero, also one whose lowest byte is zero."""
+    a = _matrix('dense', 40)
+    sel = (np.arange(40) % 3 == 1).astype(np.int32)
+    t, q = _schur(a, sel)
+    t2, q2 = _schur(a, sel * value)
+    assert np.array_equal(t, t2) and np.array_equal(q, q2)
