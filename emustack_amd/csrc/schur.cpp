@@ -42,9 +42,6 @@ inline double abs1(cplx z) { return std::fabs(z.real()) + std::fabs(z.imag()); }
 inline cplx mul(cplx a, cplx b) {
   return cplx(a.real() * b.real() - a.imag() * b.imag(), a.real() * b.imag() + a.imag() * b.real());
 }
-inline cplx mulc(cplx a, cplx b) {  // conj(a) b
-  return cplx(a.real() * b.real() + a.imag() * b.imag(), a.real() * b.imag() - a.imag() * b.real());
-}
 
 // [c s; -conj(s) c] [a; b] = [r; 0]: c = |a|^2 / d, s = a conj(b) / d, r = a (|a|^2 + |b|^2) / d with
 // d = |a| sqrt(|a|^2 + |b|^2), one square root and one division
@@ -770,7 +767,8 @@ static bool qr_entry(int n, cplx *H, int ldh, cplx *Z, int ldz, int nz) {
 #pragma clang attribute pop
 
 bool schur_available() {
-  return __builtin_cpu_supports("avx512f") && __builtin_cpu_supports("avx512dq") && __builtin_cpu_supports("avx512vl");
+  return __builtin_cpu_supports("avx512f") && __builtin_cpu_supports("avx512dq") &&
+         __builtin_cpu_supports("avx512vl") && __builtin_cpu_supports("fma");
 }
 void schur_reduce(int n, std::complex<double> *A, int lda, std::complex<double> *Q, int ldq) {
   hessenberg(n, Mat{A, lda}, Mat{Q, ldq});

@@ -5,6 +5,8 @@ the sizes where the code changes path: blocks that the small solver finishes
 strips of eight; and the shapes the eigensolver makes (a triangular part, a
 spike, a band below the diagonal)."""
 import ctypes
+import os
+import re
 
 import numpy as np
 import pytest
@@ -87,3 +89,14 @@ def test_any_nonzero_selects(value):
     t, q = _schur(a, sel)
     t2, q2 = _schur(a, sel * value)
     assert np.array_equal(t, t2) and np.array_equal(q, q2)
+
+
+def test_every_instruction_set_in_use_is_asked_for():
+    """The code is compiled for a list of CPU features; schur_available has to
+    ask for each of them (a virtual machine can mask any one)."""
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), '..', 'emustack_amd', 'csrc', 'schur.cpp')
+    with open(src) as f:
+        text = f.read()
+    used = re.search(r'target\("([^"]*)"\)', text).group(1).split(',')
+    asked = re.findall(r'__builtin_cpu_supports\("([^"]*)"\)', text)
+    assert sorted(used) == sorted(asked)
