@@ -320,6 +320,8 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
     small.resize(o_np + (np.size() + 1) / 2);
     std::memcpy(&small[o_np], np.data(), sizeof(int32_t) * np.size());
   }
+  const int nflux = L;  // down[0..L-1]
+  std::vector<zd> down((size_t)nflux * nb), upv(nb);
   double *dsmall = c->buf<double>("cs_small", small.size());
   EMU_HIP(hipMemcpyAsync(dsmall, small.data(), sizeof(double) * small.size(), hipMemcpyHostToDevice, s));
   auto part = [&](size_t at) { return reinterpret_cast<zd *>(dsmall + at); };
@@ -332,7 +334,9 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
   struct Uploads {
     hipStream_t main, st = nullptr;
     hipEvent_t ev = nullptr;
-    ~Uploads() {  // nothing reads the caller's arrays (or `small`) after the call, thrown out of or not
+    // nothing reads or writes the caller's arrays or the vectors above (declared before, so they go after this)
+    // once the call is left, thrown out of or not
+    ~Uploads() {
       (void)hipStreamSynchronize(main);
       if (st) (void)hipStreamSynchronize(st);
       if (ev) (void)hipEventDestroy(ev);
@@ -486,7 +490,6 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
   air_gap(L - 1);
   (void)rd;
   // 3. fluxes (stack.py:285-427)
-  const int nflux = L;  // down[0..L-1]
   zd *dflux = c->buf<zd>("cs_down", (size_t)nflux * nb);
   zd *uflux = c->buf<zd>("cs_up", nb);
   auto matvec = [&](const zd *M, int r, int k, const zd *v, zd *out) {
@@ -528,7 +531,6 @@ void star_cascade(Ctx *c, const CascadeArgs &a) {
   // the nets go down after the flux kernels are queued
   if (a.R_net) EMU_HIP(hipMemcpyAsync(a.R_net, rnet, sizeof(zd) * nb * d * d, hipMemcpyDeviceToHost, s));
   if (a.T_net) EMU_HIP(hipMemcpyAsync(a.T_net, tnet, sizeof(zd) * nb * d * d, hipMemcpyDeviceToHost, s));
-  std::vector<zd> down((size_t)nflux * nb), upv(nb);
   EMU_HIP(hipMemcpyAsync(down.data(), dflux, sizeof(zd) * down.size(), hipMemcpyDeviceToHost, s));
   EMU_HIP(hipMemcpyAsync(upv.data(), uflux, sizeof(zd) * nb, hipMemcpyDeviceToHost, s));
   EMU_HIP(hipStreamSynchronize(s));
