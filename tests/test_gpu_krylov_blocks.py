@@ -31,3 +31,29 @@ def test_gram_schmidt_sizes(gpu_ctx, mesh600, reference, block, ncv, lights):  #
         # both are converged to 1e-12 or better; the bounds of the comparison with the oracle
         np.testing.assert_allclose(beta[b], bref[0], rtol=1e-9, atol=1e-9 * np.abs(bref[0]).max())
         assert np.abs(J[b] @ Jd[b] - Pref).max() <= 1e-8 * np.abs(Pref).max()
+
+
+@pytest.fixture(scope='module')
+def spectrum(gpu_ctx, mesh600):  # noqa: F811
+    """24 lights, each with its own wavelength, angle and index, solved alone."""
+    mh, _ = mesh600
+    ps = [_params(480.0 + 17.0 * i, 600., 2.2 + 0.06 * i + 0.01j, 5.0 + 1.3 * i, 31.0) for i in range(24)]
+    return ps, [gpu_ctx.calc_modes_batch(mh, [p[0]], 40, 1, [p[2]], [p[3]], [p[4]], 5, block=8) for p in ps]
+
+
+@pytest.mark.parametrize('block,lights', [(1, 5), (1, 24), (2, 7), (4, 7), (4, 24), (8, 24), (0, 7)])
+def test_lights_of_a_batch_are_their_own(gpu_ctx, mesh600, spectrum, block, lights):  # noqa: F811
+    """Every light of a batch against itself alone: the instances differ, so
+    data read across them shows, and they converge after different numbers of
+    restarts, so the active ones move to other slots on the way."""
+    mh, _ = mesh600
+    ps, alone = spectrum
+    pick = [23 - i for i in range(lights)]
+    col = lambda k: [ps[i][k] for i in pick]
+    beta, J, Jd, _ = gpu_ctx.calc_modes_batch(mh, col(0), 40, 1, col(2), col(3), col(4), 5, block=block)
+    for b, i in enumerate(pick):
+        bref, Jref, Jdref, _ = alone[i]
+        # the bounds of test_gram_schmidt_sizes, for the same reason
+        np.testing.assert_allclose(beta[b], bref[0], rtol=1e-9, atol=1e-9 * np.abs(bref[0]).max())
+        Pref = Jref[0] @ Jdref[0]
+        assert np.abs(J[b] @ Jd[b] - Pref).max() <= 1e-8 * np.abs(Pref).max()
