@@ -57,12 +57,12 @@ FIXTURE = os.path.join(ROOT, 'tests', 'golden', 'configs', 'config3.npz')
 # default step), each scaled by what the counter reads for a plain 2 GiB copy;
 # summary and commands in profiles/kernels_stacked_gratings_8k.md.
 TRAFFIC_PER_DISPATCH = {
-    'k_atb_mfma16<true>': 7475500000,
-    'k_combine<16>': 7323900000,
-    'k_fwd': 433500000,
-    'k_bwd': 412900000,
-    'k_spmm_il': 2810600000,
-    'k_zgemm_nn_tall': 3957700000,
+    'k_atb_mfma16': 7466000000,
+    'k_combine<16, 1, false>': 7321000000,
+    'k_fwd': 423000000,
+    'k_bwd': 384000000,
+    'k_spmm_il<8>': 2822000000,
+    'k_zgemm_nn_tall': 3949000000,
 }
 TRAFFIC_SOURCE = 'profiles/kernels_stacked_gratings_8k.md'
 
@@ -502,8 +502,8 @@ def main():
     dom = max(prof, key=lambda k: prof[k][1])
     cnt, ms, byt = prof[dom]
     achieved = byt / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
-    kernel_name = {'solve_fwd': 'k_fwd', 'solve_bwd': 'k_bwd', 'gs_project': 'k_atb_mfma16<true>',
-                   'gs_update': 'k_combine<16>', 'spmv_M': 'k_spmm_il'}[dom]
+    kernel_name = {'solve_fwd': 'k_fwd', 'solve_bwd': 'k_bwd', 'gs_project': 'k_atb_mfma16',
+                   'gs_update': 'k_combine<16, 1, false>', 'spmv_M': 'k_spmm_il<8>'}[dom]
     m = args.ncv or 2 * NUM_BMS + NUM_BMS // 2 + 3
     m = ((m + 7) // 8) * 8
     keep = min(m - 8, NUM_BMS + (m - NUM_BMS) // 2)

@@ -1527,10 +1527,16 @@ void calc_modes(Ctx *c, DevMesh &dm, const ModesArgs &a) {
   // the basis among more columns.  Whole solves with blocks of 8 / 4 / 2, ms:
   // n = 6 k unknowns, 1 light 46 / 40 / 40, 8 lights 86 / 68 / 67; 18 k, 2
   // lights 118 / 100 / 106, 8 lights 260 / 192 / 239; 96 k, 1 light 404 / 383 /
-  // 522, 4 lights 808 / 803 / 1209.
-  // Calls that fill the card by themselves (8 lights at 96 k: 16 factors) keep
-  // 8: four such calls at once are bound by the factors' bytes and solve 3.27
-  // wavelengths per second with 8 columns, 2.82 with 4.
+  // 522, 2 lights 514 / 488, 4 lights 808 / 803 / 1209.  The line, 2 nl neq = 400 k,
+  // lies where 8 and 4 meet for a call alone.  Above it a call is mostly one of
+  // several that fill the card, and those are bound by the factors' bytes: four
+  // calls of 8 lights at once solve 3.27 wavelengths per second with 8 columns,
+  // 2.82 with 4.  Smaller calls beside others want 8 as well (lights per second,
+  // 8 / 4 columns: 96 k unknowns, 2 lights a call, two callers 6.1 / 5.8, four
+  // 7.4 / 6.3; 36 k, 5 lights, four callers 32.2 / 27.5; 12 k, 4 lights, four
+  // callers 93 / 96), but the rule sees its own call only: what other threads do
+  // should not decide how a call rounds.  A program that keeps the card full
+  // names 8.
   // The dimension and what it is refused for are those of 8-column blocks.
   const int bq = a.block > 0 ? (int)a.block : (int64_t)nb * n < 400000 ? 4 : 8;
   const int wide = a.block > 0 ? bq : 8;
